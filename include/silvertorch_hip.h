@@ -71,7 +71,8 @@ uint64_t st_murmur_hash3_2x64(uint64_t x, uint64_t y, uint64_t seed);
  *
  *   feature_offsets   device int64[num_docs * num_features + 1]
  *   bundle_b_offsets  device int64[ceil(num_docs / 2048) + 1]      (output)
- *   stats             device int64[6]                              (output)
+ *   stats             int64[6], in device memory or in pinned host memory
+ *                     that the device can write                    (output)
  *                     stats[0] = total rows (bundle_b_offsets[last]),
  *                     stats[1] = largest single-bundle width,
  *                     stats[2] = 1 if feature_offsets ever decreases, else 0,

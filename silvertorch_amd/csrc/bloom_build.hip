@@ -9,17 +9,18 @@
 //                   checks that feature_offsets never decreases.
 //   scan_kernel     one workgroup: exclusive prefix sum of the widths into
 //                   bundle_b_offsets, plus the totals the host needs.
-//   scatter_kernel  one workgroup per bundle: zeroes a b x 32-word tile in
-//                   LDS, hashes every (doc, feature, value) term of the bundle
-//                   (one thread per value, its doc and feature from an LDS
-//                   map of the slot group), ORs its k bits into the tile with
-//                   LDS atomics and writes the tile out with coalesced stores.
-//                   Bundles of up to kBuildSliceRows rows go in four passes of
-//                   512 docs, each over a b x 8-word tile (the docs' columns);
-//                   wider ones OR straight into global memory.
+//   scatter_kernel  one workgroup per part of a bundle (16 of its 32 columns,
+//                   fewer for wide bundles or few docs): clears a tile of b
+//                   rows in LDS, hashes every (doc, feature, value) term of
+//                   the part (one thread per value, its place from an LDS map
+//                   of the slot group), ORs its k bits into the tile with LDS
+//                   atomics and stores the tile.  Bundles wider than any tile
+//                   OR straight into global memory.
 // The reference's per-doc byte signatures and 64-way transpose
 // (bloom_indexer_cuda.cu:137-251, ~N*b/8 bytes of scratch) are not needed.
 #include <hip/hip_runtime.h>
+
+#include <mutex>
 
 #include "st_common.hpp"
 #include "st_errors.hpp"
@@ -29,24 +30,26 @@ int cu_count();
 
 namespace {
 
-constexpr int kWidthThreads = 256;
+constexpr int kWidthThreads = 256;        // of a bundle, many bundles
+constexpr int kWidthThreadsFew = 1024;    // of a bundle, few bundles
 constexpr int kScanThreads = 1024;
-constexpr int kBuildThreads = 1024;
-constexpr int kBuildTileRows = 512;
-constexpr int kBuildTileWords = kBuildTileRows * 32;
-constexpr int kBuildSliceRows = kBuildTileWords / 8;  // rows of a 8-column slice tile
-constexpr int kBuildSlices = 4;                       // 512-doc passes of a sliced bundle
-constexpr int kBuildFeatureCache = 256;  // murmur_mix_x of the first feature ids, in LDS
-constexpr int kBuildValueMap = 7168;     // values of a slot group mapped to their slot in LDS
+constexpr int kBuildThreads = 1024;     // of a workgroup that takes a whole CU
+constexpr int kBuildHalfThreads = 512;  // of two workgroups that share one
+constexpr int kLdsBytes = 160 * 1024;
+constexpr int kBuildFeatureCache = 64;     // murmur_mix_x of the first feature ids, in LDS
+constexpr int kBuildMapBytes = 12288;      // the places of a window's values, in LDS
+constexpr int kBuildMapFeatures = 1 << 20; // features that a 32-bit place names
+constexpr int kBuildQueueWords = 2 * 64;   // a wave's queue of values with colliding positions, in LDS
+constexpr int kBuildStaticLds = 64;        // BundleMod and alignment
+constexpr int kBuildNarrow = 1024;         // mean rows of narrow bundles
 
-// stats layout (device int64[6]):
+// stats layout (int64[6]):
 //   [0] total rows  [1] max bundle width  [2] non-decreasing violation flag
 //   [3] feature_offsets[0]  [4] feature_offsets[N*F]  [5] reserved
-constexpr int kStatsLen = 6;
 
-__global__ void init_stats_kernel(int64_t* __restrict__ stats) {
-  if (threadIdx.x < kStatsLen) stats[threadIdx.x] = 0;
-}
+// 64-bit min / max (the device library's overloads go through doubles).
+__device__ __forceinline__ int64_t lesser(int64_t a, int64_t b) { return a < b ? a : b; }
+__device__ __forceinline__ int64_t greater(int64_t a, int64_t b) { return a > b ? a : b; }
 
 __device__ __forceinline__ int64_t wave_max(int64_t v) {
 #pragma unroll
@@ -59,48 +62,58 @@ __device__ __forceinline__ int64_t wave_max(int64_t v) {
 
 // Feature counts up to this stage a chunk's offsets in LDS (below).
 constexpr int kWidthStageFeatures = 16;
+constexpr int kWidthFewFeatures = 7;  // 1,024 docs' offsets within 64 KB of LDS
 
-__global__ __launch_bounds__(kWidthThreads) void widths_kernel(
+// Marks a bundle whose offsets decrease somewhere, in the sign of its width.
+constexpr int64_t kDecreasing = INT64_MIN;
+
+// One workgroup of T threads per bundle.  256 threads keep eight workgroups on
+// a CU when there are many bundles; with fewer bundles than would fill the
+// chip so, 1,024 threads take a bundle in a quarter of the dependent steps
+// (100,000 docs of 2 features, 49 bundles: 12.3 against 6.1 us).
+template <int T>
+__global__ __launch_bounds__(T) void widths_kernel(
     const int64_t* __restrict__ offsets, int64_t num_docs, int64_t num_features,
-    int64_t k, double b_multiplier, int64_t* __restrict__ bundle_b_offsets,
-    int64_t* __restrict__ stats) {
-  __shared__ int64_t red[kWidthThreads / 64];
-  __shared__ int64_t stage[kWidthThreads * kWidthStageFeatures + 1];
+    int64_t k, double b_multiplier, int64_t* __restrict__ bundle_b_offsets) {
+  extern __shared__ __attribute__((aligned(16))) int64_t stage[];  // T * F + 1 up to 16 features
+  __shared__ int64_t red[T / 64];
+  __shared__ int any_bad;
   const int64_t bundle = blockIdx.x;
   const int64_t doc0 = bundle * kDocsPerBundle;
-  const int64_t doc1 = min(doc0 + kDocsPerBundle, num_docs);
+  const int64_t doc1 = lesser(doc0 + kDocsPerBundle, num_docs);
   const int64_t F = num_features;
+  if (threadIdx.x == 0) any_bad = 0;
   int bad = 0;
   int64_t best = 0;
   if (F <= kWidthStageFeatures) {
-    // Chunks of kWidthThreads docs: the chunk's offsets (F per doc and the
-    // next doc's first) are loaded once with coalesced loads into registers,
-    // the next chunk's loads are issued before this chunk is evaluated, and
-    // the values pass through LDS so that thread t can check that its doc's
-    // offsets never decrease and take its count from the first and the last.
-    constexpr int kPer = kWidthStageFeatures + 1;  // ns <= kPer * kWidthThreads
+    // Chunks of T docs: the chunk's offsets (F per doc and the next doc's
+    // first) are loaded once with coalesced loads into registers, the next
+    // chunk's loads are issued before this chunk is evaluated, and the values
+    // pass through LDS so that thread t can check that its doc's offsets never
+    // decrease and take its count from the first and the last.
+    constexpr int kPer = kWidthStageFeatures + 1;  // ns <= kPer * T
     int64_t r[kPer];
     const auto load = [&](int64_t c0) {
-      const int64_t ns = min<int64_t>(kWidthThreads, doc1 - c0) * F + 1;
+      const int64_t ns = lesser(T, doc1 - c0) * F + 1;
       const int64_t* src = offsets + c0 * F;
 #pragma unroll
       for (int u = 0; u < kPer; ++u) {
-        const int64_t i = threadIdx.x + u * kWidthThreads;
+        const int64_t i = threadIdx.x + u * T;
         r[u] = i < ns ? src[i] : 0;
       }
     };
     if (doc0 < doc1) load(doc0);
-    for (int64_t c0 = doc0; c0 < doc1; c0 += kWidthThreads) {
-      const int64_t nd = min<int64_t>(kWidthThreads, doc1 - c0);
+    for (int64_t c0 = doc0; c0 < doc1; c0 += T) {
+      const int64_t nd = lesser(T, doc1 - c0);
       const int64_t ns = nd * F + 1;
       __syncthreads();  // the previous chunk's readers are done with stage
 #pragma unroll
       for (int u = 0; u < kPer; ++u) {
-        const int64_t i = threadIdx.x + u * kWidthThreads;
+        const int64_t i = threadIdx.x + u * T;
         if (i < ns) stage[i] = r[u];
       }
       __syncthreads();
-      if (c0 + kWidthThreads < doc1) load(c0 + kWidthThreads);
+      if (c0 + T < doc1) load(c0 + T);
       if (threadIdx.x < nd) {
         const int64_t* o = stage + threadIdx.x * F;
         for (int64_t f = 0; f < F; ++f) bad |= o[f + 1] < o[f];
@@ -111,84 +124,158 @@ __global__ __launch_bounds__(kWidthThreads) void widths_kernel(
   } else {
     // Wide docs: every offset is read once for the monotonicity check, the
     // doc boundaries again for the counts (L2 hits).
-    for (int64_t s = doc0 * F + threadIdx.x; s < doc1 * F; s += kWidthThreads)
+    for (int64_t s = doc0 * F + threadIdx.x; s < doc1 * F; s += T)
       bad |= offsets[s + 1] < offsets[s];
-    for (int64_t d = doc0 + threadIdx.x; d < doc1; d += kWidthThreads) {
+    for (int64_t d = doc0 + threadIdx.x; d < doc1; d += T) {
       const int64_t cnt = offsets[(d + 1) * F] - offsets[d * F];
       best = cnt > best ? cnt : best;
     }
+    __syncthreads();  // any_bad is set
   }
   best = wave_max(best);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
-  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(reinterpret_cast<unsigned long long*>(stats + 2), 1ull);
+  if (__any(bad) && (threadIdx.x & 63) == 0) any_bad = 1;
   __syncthreads();
   if (threadIdx.x == 0) {
     int64_t m = red[0];
-    for (int i = 1; i < kWidthThreads / 64; ++i) m = red[i] > m ? red[i] : m;
+    for (int i = 1; i < T / 64; ++i) m = red[i] > m ? red[i] : m;
     const int64_t b = static_cast<int64_t>(static_cast<double>(m * k) * b_multiplier);
-    bundle_b_offsets[bundle + 1] = b;
-    atomicMax(reinterpret_cast<unsigned long long*>(stats + 1),
-              static_cast<unsigned long long>(b < 0 ? 0 : b));
+    bundle_b_offsets[bundle + 1] = any_bad ? (b | kDecreasing) : b;
   }
 }
 
-// In-place exclusive scan: on entry bundle_b_offsets[i+1] holds width i.
+// In-place exclusive scan: on entry bundle_b_offsets[i+1] holds width i (its
+// sign set where the bundle's offsets decrease).  The stats are stored once,
+// with plain stores: they may lie in host memory that the device can write.
 __global__ __launch_bounds__(kScanThreads) void scan_kernel(
     const int64_t* __restrict__ offsets, int64_t num_slots, int64_t nb,
     int64_t* __restrict__ bundle_b_offsets, int64_t* __restrict__ stats) {
-  __shared__ int64_t part[kScanThreads];
+  __shared__ int64_t part[kScanThreads / 64];
+  __shared__ int64_t wide[kScanThreads / 64];
+  __shared__ int any_bad;
   const int t = threadIdx.x;
   const int64_t per = (nb + kScanThreads - 1) / kScanThreads;
-  const int64_t lo = min<int64_t>(t * per, nb);
-  const int64_t hi = min<int64_t>(lo + per, nb);
-  int64_t sum = 0;
-  for (int64_t i = lo; i < hi; ++i) sum += bundle_b_offsets[i + 1];
-  part[t] = sum;
-  __syncthreads();
-  for (int off = 1; off < kScanThreads; off <<= 1) {
-    const int64_t v = t >= off ? part[t - off] : 0;
-    __syncthreads();
-    part[t] += v;
-    __syncthreads();
-  }
-  int64_t run = t == 0 ? 0 : part[t - 1];
+  const int64_t lo = lesser(t * per, nb);
+  const int64_t hi = lesser(lo + per, nb);
+  if (t == 0) any_bad = 0;
+  int64_t sum = 0, most = 0;
+  bool bad = false;
+#pragma unroll 8
   for (int64_t i = lo; i < hi; ++i) {
-    run += bundle_b_offsets[i + 1];
+    const int64_t v = bundle_b_offsets[i + 1];
+    const int64_t b = v & ~kDecreasing;
+    bad |= v < 0;
+    most = greater(most, b);
+    sum += b;
+  }
+  // inclusive scan within the wave, then over the waves
+  int64_t incl = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int64_t v = __shfl_up(incl, off, 64);
+    if ((t & 63) >= off) incl += v;
+  }
+  most = wave_max(most);
+  if ((t & 63) == 63) part[t >> 6] = incl;
+  if ((t & 63) == 0) wide[t >> 6] = most;
+  __syncthreads();
+  if (__any(bad) && (t & 63) == 0) any_bad = 1;
+  int64_t before = 0, total = 0;
+  for (int w = 0; w < kScanThreads / 64; ++w) {
+    if (w < (t >> 6)) before += part[w];
+    total += part[w];
+    most = greater(most, wide[w]);
+  }
+  __syncthreads();
+  int64_t run = before + incl - sum;
+#pragma unroll 8
+  for (int64_t i = lo; i < hi; ++i) {
+    run += bundle_b_offsets[i + 1] & ~kDecreasing;
     bundle_b_offsets[i + 1] = run;
   }
   if (t == 0) {
     bundle_b_offsets[0] = 0;
-    stats[0] = part[kScanThreads - 1];
+    stats[0] = total;
+    stats[1] = most;
+    stats[2] = any_bad;
     stats[3] = offsets[0];
     stats[4] = offsets[num_slots];
+    stats[5] = 0;
   }
 }
+
+// h mod d of a 64-bit hash for a bundle width d < 2^15, without a correction
+// step: h / d = hi * (2^32 / d) + lo * (1 / d), and only the fraction of that
+// sum matters, in 32 bits.  a ~ frac(2^32 / d) and b ~ 1 / d, rounded up, in
+// 64 fraction bits; frac = top 32 bits of hi * a + lo * b (mod 1) plus 2 for the
+// two truncated products lies above r / d by less than (d + 4) / 2^32, so
+// floor(frac * d / 2^32) is the remainder r itself while d^2 < 2^31.  Five
+// 32-bit multiplies and three adds against the general form's seven multiplies
+// and two compare-and-subtract corrections.
+struct BundleMod {
+  uint32_t d, a_lo, a_hi, b_lo, b_hi;
+};
+constexpr int64_t kBundleModMax = 1 << 15;
+
+__device__ __forceinline__ BundleMod make_bundle_mod(uint32_t d) {
+  const uint64_t q = make_fastmod_dev(d).magic;  // floor((2^64 - 1) / d)
+  const uint64_t r = 0ull - q * d;               // 2^64 = q d + r, 0 < r <= d
+  const uint32_t c = static_cast<uint32_t>((1ull << 32) % d);
+  // c * 2^64 / d = c q + c r / d <= c q + r; at most d units of 2^-64 too large
+  const uint64_t a = c == 0 ? 0 : c * q + r;
+  const uint64_t b = q + 1;
+  return {d, static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b),
+          static_cast<uint32_t>(b >> 32)};
+}
+
+__device__ __forceinline__ uint32_t bundle_mod(uint64_t h, const BundleMod& m) {
+  const uint32_t lo = static_cast<uint32_t>(h), hi = static_cast<uint32_t>(h >> 32);
+  const uint32_t frac = __umulhi(hi, m.a_lo) + hi * m.a_hi + (__umulhi(lo, m.b_lo) + lo * m.b_hi) + 2u;
+  uint32_t r = __umulhi(frac, m.d);
+  asm("" : "+v"(r));  // a 32-bit value from here on (not a shifted 64-bit product)
+  return r;
+}
+
+// The term's row position under one seed: a bundle in an LDS tile uses
+// BundleMod, one that ORs into global memory the general form.
+struct TileMod {
+  BundleMod m;
+  __device__ __forceinline__ uint32_t operator()(uint64_t h) const { return bundle_mod(h, m); }
+};
+struct WideMod {
+  FastMod64 m;
+  __device__ __forceinline__ uint32_t operator()(uint64_t h) const {
+    return static_cast<uint32_t>(fast_mod(h, m));
+  }
+};
 
 // First K distinct positions murmur(fid, value, seed) % b over seeds
 // 0, 1, 2, ... (assign_one_bits_position, bloom_index_util.cuh:183-207).
 // b >= K always holds for bundles that have terms (b >= floor(K *
-// b_multiplier) >= K), so the loop ends.
-// The first K seeds are hashed unrolled with constant seeds and compared
-// pairwise; only when two of them collide (about K^2 / 2b of the keys) does
-// the key keep the first occurrence of each position, in seed order, and go
-// on with seeds K, K + 1, ... as the sequential search would.
-template <int K>
-__device__ __forceinline__ void build_positions(uint64_t mx, uint64_t my,
-                                                const FastMod64& fm,
-                                                uint32_t (&found)[K]) {
-  // The seed-independent rotations once per key; seeds stay far below
-  // 2^27 (k distinct positions out of b >= k need few more than k seeds).
-  const uint64_t rx = rotl64(mx, 27), ry = rotl64(my, 31);
-  const bool small = fm.d < (1ull << 30);
+// b_multiplier) >= K), so the loop ends.  The first K seeds are hashed
+// unrolled with constant seeds; only when two of them collide (about K^2 / 2b
+// of the keys) does the key go on with seeds K, K + 1, ...  rx and ry are the
+// feature's and the value's halves of the hash, rotated once per key
+// (rotl(mx, 27), rotl(my, 31)); seeds stay far below 2^27 (k distinct positions
+// out of b >= k need few more than k seeds).
+
+// The positions of seeds 0 .. K - 1; true when they are distinct.
+template <int K, typename Mod>
+__device__ __forceinline__ bool first_positions(uint64_t rx, uint64_t ry, const Mod& mod, uint32_t (&found)[K]) {
   bool distinct = true;
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    const uint64_t h = murmur_finish_rot(rx, ry, static_cast<uint64_t>(j));
-    found[j] = small ? fast_mod_small(h, fm) : static_cast<uint32_t>(fast_mod(h, fm));
+  for (int j = 0; j < K; ++j) found[j] = mod(murmur_finish_rot(rx, ry, static_cast<uint64_t>(j)));
+#pragma unroll
+  for (int j = 0; j < K; ++j)
 #pragma unroll
     for (int i = 0; i < j; ++i) distinct &= found[i] != found[j];
-  }
-  if (distinct) return;
+  return distinct;
+}
+
+// first_positions' K positions with repetitions: the first occurrence of each,
+// in seed order, then further seeds' as the sequential search takes them.
+template <int K, typename Mod>
+__device__ __forceinline__ void further_positions(uint64_t rx, uint64_t ry, const Mod& mod, uint32_t (&found)[K]) {
   uint32_t first[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) first[j] = found[j];
@@ -207,9 +294,10 @@ __device__ __forceinline__ void build_positions(uint64_t mx, uint64_t my,
   }
   uint64_t seed = K;
   while (cnt < K) {
-    const uint64_t h = seed < (1ull << 27) ? murmur_finish_rot(rx, ry, seed) : murmur_finish(mx, my, seed);
+    const uint64_t h = seed < (1ull << 27) ? murmur_finish_rot(rx, ry, seed)
+                                           : murmur_finish(rotl64(rx, 37), rotl64(ry, 33), seed);
     ++seed;
-    const uint32_t p = small ? fast_mod_small(h, fm) : static_cast<uint32_t>(fast_mod(h, fm));
+    const uint32_t p = mod(h);
     bool dup = false;
 #pragma unroll
     for (int j = 0; j < K; ++j) dup |= (j < cnt) && (found[j] == p);
@@ -222,6 +310,33 @@ __device__ __forceinline__ void build_positions(uint64_t mx, uint64_t my,
   }
 }
 
+// set(p) for each of the term's k positions p.
+template <int K, typename Mod, typename Set>
+__device__ __forceinline__ void scatter_value(int64_t k, uint64_t rx, int64_t value, const Mod& mod, Set set) {
+  const uint64_t my = murmur_mix_y(static_cast<uint64_t>(value));
+  if constexpr (K > 0) {
+    const uint64_t ry = rotl64(my, 31);
+    uint32_t found[K];
+    if (!first_positions<K>(rx, ry, mod, found)) further_positions<K>(rx, ry, mod, found);
+#pragma unroll
+    for (int j = 0; j < K; ++j) set(found[j]);
+  } else {  // k above the templated range (k <= 64)
+    const uint64_t mx = rotl64(rx, 37);
+    uint32_t found[kMaxBuildK];
+    int cnt = 0;
+    uint64_t seed = 0;
+    while (cnt < k) {
+      const uint32_t p = mod(murmur_finish(mx, my, seed++));
+      bool dup = false;
+      for (int j = 0; j < cnt; ++j) dup |= found[j] == p;
+      if (!dup) found[cnt++] = p;
+    }
+    for (int j = 0; j < k; ++j) set(found[j]);
+  }
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 struct ScatterArgs {
   const int32_t* feature_ids;
   const int64_t* offsets;
@@ -229,204 +344,261 @@ struct ScatterArgs {
   int64_t num_values;
   int64_t num_features;
   int64_t num_docs;
+  int64_t num_bundles;
   int64_t k;
   const int64_t* bundle_b_offsets;
   unsigned long long* index;
+  int lc;         // a workgroup's part of a bundle: 2^lc columns (64 * 2^lc docs)
+  int tile_rows;  // rows its LDS tile holds
 };
 
-// Swizzled LDS word of a tile of 2^lc columns (row p, column c): spreads the
-// 64 lanes of a wave, which mostly share a column, over the LDS banks.
-__device__ __forceinline__ int tile_word(uint32_t p, uint32_t c, int lc) {
-  return static_cast<int>((p << lc) + (c ^ (p & ((1u << lc) - 1u))));
+// A tile row: the part's columns as 32-bit words, one word of padding so that
+// the rows' words of one column lie on different LDS banks (64 lanes mostly
+// share a column and differ in the row).
+__host__ __device__ constexpr int tile_stride(int lc) { return (2 << lc) + 1; }
+
+// A value's place, as the slot threads record it in the value map: the doc's
+// bit (doc % 32) in bits 0-4, its 32-bit word in a tile row in bits 5-9 (the
+// high half of a 64-bit column, docs 0-31, is the odd word), the feature above:
+// 16 bits hold the first kBuildFeatureCache features, 32 bits the first
+// kBuildMapFeatures.
+__device__ __forceinline__ uint32_t place(uint32_t d, uint32_t f, uint32_t c0) {
+  return (d & 31u) | ((((d >> 5) ^ 1u) - 2 * c0) << 5) | (f << 10);
 }
+__device__ __forceinline__ uint32_t place_bit(uint32_t m) { return 0x80000000u >> (m & 31u); }
+__device__ __forceinline__ uint32_t place_word(uint32_t m) { return (m >> 5) & 31u; }
+__device__ __forceinline__ uint32_t place_feature(uint32_t m) { return m >> 10; }
 
-// Sets the term's bits either in the LDS tile or in global memory.
-template <int K>
-__device__ __forceinline__ void scatter_term(const ScatterArgs& a, int lc,
-                                             unsigned long long* tile,
-                                             unsigned long long* gbase,
-                                             const FastMod64& fm, uint64_t mx,
-                                             uint64_t my, uint32_t col,
-                                             unsigned long long bit) {
-  uint32_t found[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) found[j] = 0;
-  build_positions<K>(mx, my, fm, found);
-#pragma unroll
-  for (int j = 0; j < K; ++j) {
-    if (lc >= 0) {
-      atomicOr(tile + tile_word(found[j], col, lc), bit);
-    } else {
-      atomicOr(gbase + static_cast<uint64_t>(found[j]) * 32 + col, bit);
-    }
-  }
-}
-
-// Runtime-k variant for k above the templated range (k <= 64).
-__device__ void scatter_term_generic(const ScatterArgs& a, int lc,
-                                     unsigned long long* tile,
-                                     unsigned long long* gbase,
-                                     const FastMod64& fm, uint64_t mx,
-                                     uint64_t my, uint32_t col,
-                                     unsigned long long bit) {
-  uint32_t found[kMaxBuildK];
-  const int k = static_cast<int>(a.k);
-  int cnt = 0;
-  uint64_t seed = 0;
-  while (cnt < k) {
-    const uint32_t p = static_cast<uint32_t>(fast_mod(murmur_finish(mx, my, seed++), fm));
-    bool dup = false;
-    for (int j = 0; j < cnt; ++j) dup |= found[j] == p;
-    if (!dup) found[cnt++] = p;
-  }
-  for (int j = 0; j < k; ++j) {
-    if (lc >= 0) {
-      atomicOr(tile + tile_word(found[j], col, lc), bit);
-    } else {
-      atomicOr(gbase + static_cast<uint64_t>(found[j]) * 32 + col, bit);
-    }
-  }
-}
-
-template <int K>
-__device__ __forceinline__ void scatter_value(const ScatterArgs& a, int lc,
-                                              unsigned long long* tile,
-                                              unsigned long long* gbase, const FastMod64& fm,
-                                              uint64_t mx, int64_t value, uint32_t col,
-                                              unsigned long long bit) {
-  const uint64_t my = murmur_mix_y(static_cast<uint64_t>(value));
-  if constexpr (K > 0) {
-    scatter_term<K>(a, lc, tile, gbase, fm, mx, my, col, bit);
-  } else {
-    scatter_term_generic(a, lc, tile, gbase, fm, mx, my, col, bit);
-  }
-}
-
-// One workgroup per bundle.  The bundle's (doc, feature) slots go in groups
-// of kBuildThreads: each slot thread records its doc and feature for each of
-// its values in an LDS map, then the threads take the group's values one
-// each (all lanes hash, value loads coalesce).  A group with more values than
-// the map holds walks them per slot instead.  The seed-independent half of
-// the feature id's hash comes from LDS.  With one workgroup per CU nothing
-// else covers the workgroup's global-load waits, so the loads are issued a
-// step ahead: the next group's offsets during this group, the next value
-// of a thread before the current one is hashed.
-template <int K>
-__global__ __launch_bounds__(kBuildThreads) void scatter_kernel(ScatterArgs a) {
-  __shared__ unsigned long long tile[kBuildTileWords];
-  __shared__ uint64_t mxc[kBuildFeatureCache];
-  __shared__ uint32_t vmap[kBuildValueMap];  // doc | feature << 11 of each value
-
-  const int tid = threadIdx.x;
-  const int64_t bundle = blockIdx.x;
-  const int64_t start = a.bundle_b_offsets[bundle];
-  const int64_t b = a.bundle_b_offsets[bundle + 1] - start;
-  // tile columns 2^lc: the whole bundle (32), a 512-doc slice (8), or no
-  // tile (-1: bits go straight to global memory)
-  const int lc = b <= kBuildTileRows ? 5 : (b <= kBuildSliceRows ? 3 : -1);
-  const int passes = lc == 3 ? kBuildSlices : 1;
-  unsigned long long* gbase = a.index + start * 32;
-  const int64_t F = a.num_features;
-  const int64_t cached = min<int64_t>(F, kBuildFeatureCache);
-
-  for (int i = tid; i < cached; i += kBuildThreads)
-    mxc[i] = murmur_mix_x(static_cast<uint64_t>(static_cast<int64_t>(a.feature_ids[i])));
-  if (lc < 0) {
-    for (int64_t w = tid; w < b * 32; w += kBuildThreads) gbase[w] = 0;
-    __threadfence();
-  }
-  const FastMod64 fm = make_fastmod(static_cast<uint64_t>(b > 0 ? b : 1));
-  const int64_t doc0 = bundle * kDocsPerBundle;
-  const int64_t doc1 = min(doc0 + kDocsPerBundle, a.num_docs);
-  const int64_t* offs = a.offsets + doc0 * F;
-  const bool mappable = F < (1 << 21);  // doc (11 bits) and feature share a u32
-  auto mx_of = [&](int64_t f) -> uint64_t {
-    return f < cached
-               ? mxc[f]
-               : murmur_mix_x(static_cast<uint64_t>(static_cast<int64_t>(a.feature_ids[f])));
-  };
+// one(value, place, index, mine) for each value of the part's slots [slot_lo, slot_hi)
+// (slot = doc * F + feature, doc relative to the bundle).
+// Slots go in groups of kSlots per thread, a group's values in windows of
+// the map's entries, for which every slot thread records its place in an LDS map,
+// so that the threads then take the window's values one each (all lanes hash,
+// value loads coalesce).  A thread's next value is loaded before the current
+// one is hashed: the load is an atomic one of wavefront scope, an ordinary
+// load whose order the compiler keeps (a plain load it sinks to the value's
+// use, where every value waits for memory).
+template <typename Place, typename One>
+__device__ __forceinline__ void for_each_value(const ScatterArgs& a, const int64_t* offs, uint32_t c0,
+                                               int64_t slot_lo, int64_t slot_hi, Place* vmap, One one) {
+  constexpr int kSlots = 4;
+  constexpr int kWindow = kBuildMapBytes / sizeof(Place);
+  const int tid = threadIdx.x, T = blockDim.x;
+  const uint32_t F = static_cast<uint32_t>(a.num_features);
+  const uint32_t step_d = T / F, step_f = T % F;
   // Values outside [0, num_values) are never read (the host rejects offsets
   // that would point there before launching).
-  auto clampv = [&](int64_t v) { return min<int64_t>(max<int64_t>(v, 0), a.num_values); };
+  auto clampv = [&](int64_t v) { return lesser(greater(v, 0), a.num_values); };
+  const uint32_t first = static_cast<uint32_t>(slot_lo) + tid;
+  uint32_t d = first / F, f = first % F;
+  for (int64_t g = slot_lo; g < slot_hi; g += kSlots * T) {
+    int64_t v0[kSlots], v1[kSlots];
+    uint32_t at[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+      // clamped, not predicated: the loads go out together
+      const int64_t rel = g + s * T + tid;
+      const int64_t* o = offs + lesser(rel, slot_hi - 1);
+      v0[s] = o[0];
+      v1[s] = rel < slot_hi ? o[1] : o[0];
+      at[s] = place(d, f, c0);
+      d += step_d;
+      f += step_f;
+      if (f >= F) {
+        f -= F;
+        ++d;
+      }
+    }
+    const int64_t gv0 = clampv(offs[g]);
+    const int64_t gv1 = clampv(offs[lesser(g + kSlots * T, slot_hi)]);
+    for (int64_t w = gv0; w < gv1; w += kWindow) {
+      const int n = static_cast<int>(lesser(kWindow, gv1 - w));
+      const int64_t* vals = a.values + w;
+      auto load = [&](int i) {
+        const uint32_t c = static_cast<uint32_t>(i < n ? i : n - 1);
+        return __hip_atomic_load(vals + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      };
+      int64_t value = load(tid);
+      __syncthreads();  // the previous window's readers are done with vmap
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        const int lo = static_cast<int>(lesser(greater(v0[s] - w, 0), n));
+        const int hi = static_cast<int>(lesser(greater(v1[s] - w, 0), n));
+        for (int i = lo; i < hi; ++i) vmap[i] = static_cast<Place>(at[s]);
+      }
+      __syncthreads();
+      // whole waves: the last values' wave runs with its spare lanes repeating
+      // the window's last value, `mine` false
+      for (int i0 = __builtin_amdgcn_readfirstlane(tid & ~63); i0 < n; i0 += T) {
+        const int i = i0 + (tid & 63);
+        const int64_t next = load(i + T);
+        one(value, vmap[i < n ? i : n - 1], w + i, i < n);
+        value = next;
+      }
+    }
+  }
+}
 
-  for (int pass = 0; pass < passes; ++pass) {
-    // this pass's docs [dlo, dhi) (bundle-relative) and first tile column
-    const int64_t dlo = lc == 3 ? pass * (kDocsPerBundle / kBuildSlices) : 0;
-    const int64_t dhi = lc == 3 ? min<int64_t>(dlo + kDocsPerBundle / kBuildSlices, doc1 - doc0)
-                                : doc1 - doc0;
-    const uint32_t c0 = static_cast<uint32_t>(dlo >> 6);
-    const int64_t tw = lc < 0 ? 0 : (b << lc);
-    const int64_t slot_lo = dlo * F, slot_hi = max<int64_t>(dhi, dlo) * F;
-    // the offsets a group reads: its slot's two and the group's two bounds
-    struct GroupOffsets {
-      int64_t o0, o1, g0, g1;
+// One workgroup per part of a bundle (2^lc of its 32 columns).  The tile of
+// the part's rows is cleared in LDS, the part's values are hashed one per
+// thread, their bits ORed into the tile and the tile stored.  The parts of a
+// bundle lie 8 workgroups apart, on one XCD, so that the lines they share
+// meet in its L2.  Parts rather than whole bundles: two tiles fit a CU, so one
+// workgroup hashes while the other clears, loads offsets or stores, and a
+// small corpus (49 bundles at 100,000 docs) still fills the chip.
+// Bound by VALU issue: 236 wave instructions per 64 values at k = 3, one per 4.3
+// cycles (nearly every instruction of the hash, 32-bit multiplies and
+// v_mad_u64_u32 included, takes 4).  100M docs x 4 features, 1.8e9 values, 470
+// rows: 12.0 ms; 17.0 ms with a whole bundle per workgroup (one a CU), the
+// general remainder and 64-bit tile words (315 instructions).  100,000 docs x 2
+// features: 11.8 against 29.9 us.  With 24 waves a CU instead of 16 no faster.
+template <int K>
+__global__ __launch_bounds__(kBuildThreads) void scatter_kernel(ScatterArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  __shared__ BundleMod s_mod;
+  const int lc = a.lc, stride = tile_stride(lc);
+  const int tid = threadIdx.x, T = blockDim.x;
+  uint64_t* rxc = reinterpret_cast<uint64_t*>(lds);  // rotl(murmur_mix_x(id), 27)
+  uint32_t* vmap = lds + 2 * kBuildFeatureCache;
+  uint16_t* vmap16 = reinterpret_cast<uint16_t*>(vmap);
+  uint32_t* queues = vmap + kBuildMapBytes / 4;
+  uint32_t* tile = queues + kBuildQueueWords * (T >> 6);
+
+  const int parts = 32 >> lc;
+  const int64_t run = blockIdx.x / (8 * parts), at = blockIdx.x % (8 * parts);
+  const int64_t bundle = run * 8 + at % 8;
+  const int part = static_cast<int>(at / 8);
+  if (bundle >= a.num_bundles) return;
+  const int64_t start = a.bundle_b_offsets[bundle];
+  const int64_t b = a.bundle_b_offsets[bundle + 1] - start;
+  if (b <= 0) return;
+  const bool tiled = b <= a.tile_rows;
+  const uint32_t c0 = static_cast<uint32_t>(part) << lc;
+  unsigned long long* gbase = a.index + start * 32 + c0;
+  const int64_t F = a.num_features;
+  auto rx_id = [&](int64_t f) {
+    return rotl64(murmur_mix_x(static_cast<uint64_t>(static_cast<int64_t>(a.feature_ids[f]))), 27);
+  };
+
+  const int64_t words = b << lc;
+  if (tiled) {
+    for (int i = tid; i < static_cast<int>(lesser(F, kBuildFeatureCache)); i += T) rxc[i] = rx_id(i);
+    if (tid == T - 1) s_mod = make_bundle_mod(static_cast<uint32_t>(b));
+    u32x4* clear = reinterpret_cast<u32x4*>(tile);
+    for (int w = tid; w < (static_cast<int>(b) * stride + 3) / 4; w += T) clear[w] = u32x4{0, 0, 0, 0};
+  } else {
+    for (int64_t w = tid; w < words; w += T) gbase[(w >> lc) * 32 + (w & ((1 << lc) - 1))] = 0;
+    __threadfence();
+  }
+  __syncthreads();
+
+  const int64_t doc0 = bundle * kDocsPerBundle;
+  const int64_t docs = lesser(doc0 + kDocsPerBundle, a.num_docs) - doc0;
+  const int64_t dlo = static_cast<int64_t>(c0) * 64;
+  const int64_t dhi = lesser(dlo + (64 << lc), docs);
+  const int64_t* offs = a.offsets + doc0 * F;
+  const int64_t slot_lo = dlo * F, slot_hi = dhi > dlo ? dhi * F : slot_lo;
+  if (tiled && F <= kBuildFeatureCache) {
+    TileMod mod{s_mod};
+    mod.m.d = __builtin_amdgcn_readfirstlane(mod.m.d);
+    mod.m.a_lo = __builtin_amdgcn_readfirstlane(mod.m.a_lo);
+    mod.m.a_hi = __builtin_amdgcn_readfirstlane(mod.m.a_hi);
+    mod.m.b_lo = __builtin_amdgcn_readfirstlane(mod.m.b_lo);
+    mod.m.b_hi = __builtin_amdgcn_readfirstlane(mod.m.b_hi);
+    const uint32_t row_bytes = 4 * stride;
+    auto set = [&](uint32_t p, uint32_t m) {
+      atomicOr(reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(tile) +
+                                           (__umul24(p, row_bytes) + 4 * place_word(m))),
+               place_bit(m));
     };
-    auto load_group = [&](int64_t g) {
-      GroupOffsets o{0, 0, 0, 0};
-      if (g >= slot_hi) return o;
-      const int64_t rel = g + tid;
-      if (rel < slot_hi) {
-        o.o0 = offs[rel];
-        o.o1 = offs[rel + 1];
-      }
-      o.g0 = offs[g];
-      o.g1 = offs[min<int64_t>(g + kBuildThreads, slot_hi)];
-      return o;
-    };
-    // the first group's offsets are in flight while the tile is cleared
-    GroupOffsets next = load_group(b > 0 ? slot_lo : slot_hi);
-    for (int64_t w = tid; w < tw; w += kBuildThreads) tile[w] = 0;
-    __syncthreads();
-    for (int64_t g = slot_lo; b > 0 && g < slot_hi; g += kBuildThreads) {
-      const GroupOffsets cur = next;
-      next = load_group(g + kBuildThreads);
-      const int64_t rel = g + tid;
-      const bool has_slot = rel < slot_hi;
-      const int64_t v0 = has_slot ? clampv(cur.o0) : 0;
-      const int64_t v1 = has_slot ? clampv(cur.o1) : 0;
-      const int64_t d = has_slot ? rel / F : 0;
-      const int64_t f = has_slot ? rel - d * F : 0;
-      const int64_t gv0 = clampv(cur.g0);
-      const int64_t gv1 = clampv(cur.g1);
-      if (mappable && gv1 - gv0 <= kBuildValueMap) {  // uniform across the workgroup
-        // Value loads are clamped to the group's last value rather than
-        // predicated: with the same loads on every path the next value stays
-        // in flight while the current one is hashed.  The first is issued
-        // before the map is built.
-        const int64_t last = max<int64_t>(gv1 - 1, gv0);
-        const bool any = gv1 > gv0;  // uniform
-        int64_t j = gv0 + tid;
-        int64_t value = any ? a.values[min(j, last)] : 0;
-        __syncthreads();  // previous group's readers are done with vmap
-        for (int64_t i = v0; i < v1; ++i)
-          vmap[i - gv0] = static_cast<uint32_t>(d) | (static_cast<uint32_t>(f) << 11);
-        __syncthreads();
-        for (; j < gv1; j += kBuildThreads) {
-          const int64_t value_next = a.values[min(j + kBuildThreads, last)];
-          const uint32_t m = vmap[j - gv0];
-          const uint32_t dd = m & 2047u;
-          scatter_value<K>(a, lc, tile, gbase, fm, mx_of(m >> 11), value, (dd >> 6) - c0,
-                           1ull << (63 - (dd & 63)));
-          value = value_next;
+    if constexpr (K > 1) {
+      // Values whose first K positions collide (0.6% of the values, but a third
+      // of the waves hold one, at b = 470 and K = 3) wait in the wave's queue
+      // until it is full, and are then hashed again and further together.
+      uint32_t* queue = queues + (tid >> 6) * kBuildQueueWords;
+      const int lane = tid & 63;
+      const int64_t base = slot_hi > slot_lo ? lesser(greater(offs[slot_lo], 0), a.num_values) : 0;
+      int queued = 0;  // wave-uniform
+      auto drain = [&] {
+        if (lane < queued) {
+          const uint32_t i = queue[2 * lane], m = queue[2 * lane + 1];
+          scatter_value<K>(a.k, rxc[place_feature(m)], a.values[base + i], mod, [&](uint32_t p) { set(p, m); });
         }
-      } else if (v0 < v1) {
-        const uint64_t mx = mx_of(f);
-        for (int64_t j = v0; j < v1; ++j)
-          scatter_value<K>(a, lc, tile, gbase, fm, mx, a.values[j],
-                           static_cast<uint32_t>(d >> 6) - c0, 1ull << (63 - (d & 63)));
+        queued = 0;
+      };
+      for_each_value(a, offs, c0, slot_lo, slot_hi, vmap16, [&](int64_t value, uint32_t m, int64_t index, bool mine) {
+        const uint64_t rx = rxc[place_feature(m)];
+        const uint64_t ry = rotl64(murmur_mix_y(static_cast<uint64_t>(value)), 31);
+        uint32_t found[K];
+        const bool distinct = first_positions<K>(rx, ry, mod, found);
+        if (mine && distinct) {
+#pragma unroll
+          for (int j = 0; j < K; ++j) set(found[j], m);
+        }
+        const bool wait = mine && !distinct;
+        const uint64_t again = __ballot(wait);
+        if (again != 0) {
+          const int more = __popcll(again);
+          if (queued + more > 64) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            drain();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          }
+          if (wait) {
+            const int at_q = queued + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(again >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(again), 0));
+            queue[2 * at_q] = static_cast<uint32_t>(index - base);
+            queue[2 * at_q + 1] = m;
+          }
+          queued += more;
+        }
+      });
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      drain();
+    } else {
+      for_each_value(a, offs, c0, slot_lo, slot_hi, vmap16, [&](int64_t value, uint32_t m, int64_t, bool mine) {
+        if (mine) scatter_value<K>(a.k, rxc[place_feature(m)], value, mod, [&](uint32_t p) { set(p, m); });
+      });
+    }
+  } else {
+    // A bundle wider than the tile (its bits go straight to global memory),
+    // or more features than the cache or than a place names (a thread per
+    // slot then).
+    const WideMod mod{make_fastmod(static_cast<uint64_t>(b))};
+    auto one = [&](int64_t value, int64_t f, uint32_t word, uint32_t doc) {
+      scatter_value<K>(a.k, rx_id(f), value, mod, [&](uint32_t p) {
+        if (tiled) {
+          atomicOr(tile + (p * stride + word), 0x80000000u >> doc);
+        } else {
+          atomicOr(gbase + static_cast<uint64_t>(p) * 32 + (word >> 1),
+                   1ull << (((word & 1u) << 5) + 31u - doc));
+        }
+      });
+    };
+    if (F < kBuildMapFeatures) {
+      for_each_value(a, offs, c0, slot_lo, slot_hi, vmap, [&](int64_t value, uint32_t m, int64_t, bool mine) {
+        if (mine) one(value, place_feature(m), place_word(m), m & 31u);
+      });
+    } else {
+      for (int64_t rel = slot_lo + tid; rel < slot_hi; rel += T) {
+        const int64_t d = rel / F, f = rel - d * F;
+        const int64_t v0 = lesser(greater(offs[rel], 0), a.num_values);
+        const int64_t v1 = lesser(greater(offs[rel + 1], 0), a.num_values);
+        for (int64_t v = v0; v < v1; ++v)
+          one(a.values[v], f, static_cast<uint32_t>(((d >> 5) ^ 1) - 2 * c0), static_cast<uint32_t>(d & 31));
       }
     }
-    __syncthreads();
-    if (lc >= 0) {
-      const uint32_t cmask = (1u << lc) - 1u;
-      for (int64_t w = tid; w < tw; w += kBuildThreads) {
-        const uint32_t p = static_cast<uint32_t>(w >> lc);
-        const uint32_t c = static_cast<uint32_t>(w) & cmask;
-        __builtin_nontemporal_store(tile[tile_word(p, c, lc)],
-                                    gbase + static_cast<int64_t>(p) * 32 + c0 + c);
-      }
-      if (pass + 1 < passes) __syncthreads();  // the stores have read the tile
-    }
+  }
+  if (!tiled) return;
+  __syncthreads();
+  for (int w = tid; w < static_cast<int>(words); w += T) {
+    const int p = w >> lc, c = w & ((1 << lc) - 1);
+    const uint32_t* src = tile + p * stride + 2 * c;
+    const unsigned long long v = (static_cast<unsigned long long>(src[1]) << 32) | src[0];
+    unsigned long long* dst = gbase + static_cast<int64_t>(p) * 32 + c;
+    // whole 128-byte lines stream past the caches; parts of a line meet in L2
+    if (lc >= 4) __builtin_nontemporal_store(v, dst);
+    else *dst = v;
   }
 }
 
@@ -454,6 +626,57 @@ void check_launch(const char* what) {
     throw Error(ST_ERR_HIP, cat(what, " launch failed: ", hipGetErrorString(e)));
 }
 
+// The tile may take more than the 64 KB default limit.
+void set_lds_limits() {
+  static std::once_flag once;
+  static hipError_t status = hipSuccess;
+  std::call_once(once, [] {
+    for (int64_t k = 0; k <= 10; ++k) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(select_scatter(k)),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               kLdsBytes - kBuildStaticLds);
+      if (e != hipSuccess && status == hipSuccess) status = e;
+    }
+  });
+  if (status != hipSuccess)
+    throw Error(ST_ERR_HIP, cat("hipFuncSetAttribute failed: ", hipGetErrorString(status)));
+}
+
+struct ScatterShape {
+  int lc, tile_rows, threads, lds;
+};
+
+// LDS of a workgroup besides its tile.
+int fixed_lds(int threads) {
+  return 8 * kBuildFeatureCache + kBuildMapBytes + 4 * kBuildQueueWords * (threads / 64);
+}
+
+// Rows a tile holds when a workgroup of `threads` may use `lds` bytes.
+int tile_rows_in(int lds, int threads, int lc) {
+  return (lds - kBuildStaticLds - fixed_lds(threads)) / (4 * tile_stride(lc));
+}
+
+// The part of a bundle a workgroup takes: as many columns as let two tiles of
+// the widest bundle share a CU (16 columns up to 492 rows, 8 up to 955, 4 up
+// to 1,804), else as many as fit the whole CU (4 up to 3,966 rows, 2 up to
+// 7,139, 1 up to 11,898).  Where a few bundles are that wide among narrow ones
+// (mean below kBuildNarrow), the parts keep 8 columns and the bundles that no
+// tile holds OR into global memory, as bundles wider than any tile do (1M docs
+// of up to 96 values, k = 5, 3,900-4,300 rows: 11.0 ms so, 0.94 ms in 2-column
+// tiles).  A corpus too small to give every CU two workgroups is split further.
+ScatterShape scatter_shape(int64_t max_b, int64_t total_rows, int64_t nb) {
+  ScatterShape s{3, tile_rows_in(kLdsBytes, kBuildThreads, 3), kBuildThreads, 0};
+  const bool wide = total_rows >= kBuildNarrow * nb;
+  for (int lc = wide ? 0 : 2; lc <= 2; ++lc)
+    if (max_b <= tile_rows_in(kLdsBytes, kBuildThreads, lc)) s = {lc, static_cast<int>(max_b), kBuildThreads, 0};
+  for (int lc = 2; lc <= 4; ++lc)
+    if (max_b <= tile_rows_in(kLdsBytes / 2, kBuildHalfThreads, lc))
+      s = {lc, static_cast<int>(max_b), kBuildHalfThreads, 0};
+  while (s.lc > 2 && s.threads == kBuildHalfThreads && nb * (32 >> s.lc) < 2 * cu_count()) --s.lc;
+  s.lds = fixed_lds(s.threads) + (4 * tile_stride(s.lc) * s.tile_rows + 15) / 16 * 16;
+  return s;
+}
+
 }  // namespace
 }  // namespace st
 
@@ -473,12 +696,13 @@ extern "C" int st_bloom_build_bundle_offsets(const int64_t* feature_offsets,
     ST_CHECK(feature_offsets && bundle_b_offsets && stats, "null device pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t nb = (num_docs + kDocsPerBundle - 1) / kDocsPerBundle;
-    hipLaunchKernelGGL(init_stats_kernel, dim3(1), dim3(64), 0, s, stats);
-    check_launch("init_stats_kernel");
     if (nb > 0) {
-      hipLaunchKernelGGL(widths_kernel, dim3(static_cast<unsigned>(nb)),
-                         dim3(kWidthThreads), 0, s, feature_offsets, num_docs,
-                         num_features, k, b_multiplier, bundle_b_offsets, stats);
+      const int64_t staged = num_features <= kWidthStageFeatures ? num_features : 0;
+      const bool few = nb < 4 * cu_count() && staged <= kWidthFewFeatures;
+      const int threads = few ? kWidthThreadsFew : kWidthThreads;
+      hipLaunchKernelGGL(few ? widths_kernel<kWidthThreadsFew> : widths_kernel<kWidthThreads>,
+                         dim3(static_cast<unsigned>(nb)), dim3(threads), 8 * (threads * staged + 1), s,
+                         feature_offsets, num_docs, num_features, k, b_multiplier, bundle_b_offsets);
       check_launch("widths_kernel");
     }
     hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(kScanThreads), 0, s,
@@ -507,7 +731,8 @@ extern "C" int st_bloom_index_build(const int32_t* feature_ids,
     ST_CHECK(feature_ids && feature_offsets && bundle_b_offsets && bloom_index,
              "null device pointer");
     ST_CHECK(num_values == 0 || feature_values, "feature_values is null");
-    (void)max_b;
+    set_lds_limits();
+    const ScatterShape shape = scatter_shape(max_b, bloom_index_numel / kColumnsPerBundle, nb);
     ScatterArgs a;
     a.feature_ids = feature_ids;
     a.offsets = feature_offsets;
@@ -518,9 +743,13 @@ extern "C" int st_bloom_index_build(const int32_t* feature_ids,
     a.k = k;
     a.bundle_b_offsets = bundle_b_offsets;
     a.index = reinterpret_cast<unsigned long long*>(bloom_index);
+    a.num_bundles = nb;
+    a.lc = shape.lc;
+    a.tile_rows = shape.tile_rows;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(select_scatter(k), dim3(static_cast<unsigned>(nb)),
-                       dim3(kBuildThreads), 0, s, a);
+    const int64_t grid = (nb + 7) / 8 * 8 * (32 >> shape.lc);
+    hipLaunchKernelGGL(select_scatter(k), dim3(static_cast<unsigned>(grid)), dim3(shape.threads),
+                       shape.lds, s, a);
     check_launch("scatter_kernel");
   });
 }

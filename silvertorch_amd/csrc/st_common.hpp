@@ -81,11 +81,20 @@ ST_HD uint64_t murmur_pair(uint64_t x, uint64_t y, uint64_t seed) {
 // rotl(seed ^ m, r) = rotl(m, r) ^ (seed << r) (r = 27, 31), so the
 // rotations of mx and my are taken once per key (rx = rotl(mx, 27),
 // ry = rotl(my, 31)).  Equal to murmur_finish(mx, my, seed) for those seeds.
+// 5 h: on the device one shift-and-add (the compiler's multiplies by 5 take two
+// and two moves).
+ST_HD uint64_t times5(uint64_t h) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint64_t r;
+  asm("v_lshl_add_u64 %0, %1, 2, %1" : "=v"(r) : "v"(h));
+  return r;
+#else
+  return h * 5;
+#endif
+}
 ST_HD uint64_t murmur_finish_rot(uint64_t rx, uint64_t ry, uint64_t seed) {
-  uint64_t h1 = (rx ^ (seed << 27)) + seed;
-  h1 = h1 * 5 + 0x52dce729ULL;
-  uint64_t h2 = (ry ^ (seed << 31)) + h1;
-  h2 = h2 * 5 + 0x38495ab5ULL;
+  uint64_t h1 = times5(rx ^ (seed << 27)) + (seed * 5 + 0x52dce729ULL);
+  uint64_t h2 = times5((ry ^ (seed << 31)) + h1) + 0x38495ab5ULL;
   h1 ^= 16;
   h2 ^= 16;
   h1 += h2;

@@ -100,14 +100,16 @@ std::tuple<Tensor, Tensor> build_gpu(const Tensor& feature_ids_in,
 
   auto lopts = at::TensorOptions().dtype(at::kLong).device(dev);
   Tensor bundle_b_offsets = at::empty({nb + 1}, lopts);
-  Tensor stats = at::empty({6}, lopts);
+  // the index size is data dependent: the last kernel stores it straight to
+  // pinned memory, which the host reads once the stream has run
+  const Tensor stats = at::empty({6}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
   check_st(st_bloom_build_bundle_offsets(offsets.data_ptr<int64_t>(), N, F, k,
                                          b_multiplier,
                                          bundle_b_offsets.data_ptr<int64_t>(),
                                          stats.data_ptr<int64_t>(), stream),
            "bloom_index_build");
-  const Tensor st = stats.cpu();  // the index size is data dependent
-  const int64_t* s = st.data_ptr<int64_t>();
+  c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).synchronize();
+  const int64_t* s = stats.data_ptr<int64_t>();
   TORCH_CHECK(s[2] == 0, "feature_offsets must be non-decreasing");
   TORCH_CHECK(s[3] >= 0 && s[4] <= values.numel(), "feature_offsets range [",
               s[3], ", ", s[4], ") lies outside feature_values (",

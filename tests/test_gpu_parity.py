@@ -169,6 +169,35 @@ def test_build_feature_counts_vs_oracle(F, n):
                                        torch.from_numpy(vals).cuda(), 2.0, 3)
 
 
+# Widest bundle's rows on both sides of each tile limit (492, 955 and 1,804
+# rows with half a CU, 3,966, 7,139 and 11,898 with a whole one, then global
+# memory; beyond 3,966 narrow tiles only where the mean width is large: docs
+# in one or two bundles).
+@pytest.mark.parametrize("widest", [2, 492, 494, 954, 956, 1804, 1806, 3966, 3968, 7138, 7140, 11898, 11904])
+@pytest.mark.parametrize("docs,F", [(4097, 3), (4097, 64), (1500, 2), (4097, 65), (530_001, 1)])
+def test_build_tile_shapes_vs_oracle(widest, docs, F):
+    """Every split of a bundle over workgroups (by the widest bundle and by
+    the number of bundles), value counts from none to many per slot, one bundle
+    wider than the rest."""
+    k, bm = (1, 2.0) if widest % 4 else (2, 1.001)
+    rng = np.random.default_rng(widest + docs + F)
+    counts = (rng.random(docs * F) < (1.5 / F)).astype(np.int64)
+    most = -(-widest // 2)
+    doc = int(rng.integers(0, docs))  # the doc that makes its bundle the widest
+    counts.reshape(docs, F)[doc] = 0
+    at = np.sort(rng.integers(0, F, most))
+    np.add.at(counts.reshape(docs, F)[doc], at, 1)
+    offs = np.concatenate([[0], np.cumsum(counts)])
+    vals = rng.integers(-2**62, 2**62, int(offs[-1]))
+    ids = np.arange(1, F + 1, dtype=np.int32) * 7
+    H.note(f"[build tiles] widest={widest} docs={docs} F={F} k={k}")
+    index, bbo = H.build(ids, offs, vals, bm, k)
+    want_index, want_bbo = O.bloom_build(ids, offs, vals, bm, k)
+    np.testing.assert_array_equal(bbo, want_bbo)
+    np.testing.assert_array_equal(index, want_index)
+    assert int(np.diff(bbo).max()) >= widest
+
+
 def test_many_terms_split_into_passes():
     """More distinct terms than one LDS position area holds -> several passes."""
     rng = np.random.default_rng(77)
