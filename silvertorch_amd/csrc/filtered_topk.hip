@@ -47,6 +47,11 @@ constexpr int kScoreThreads = 512;   // 8 waves; one workgroup per CU
 constexpr int kScoreWaves = kScoreThreads / 64;
 constexpr int kQueryTile = 32;
 constexpr int kLdsBytes = 160 * 1024;
+// topk_score_few_kernel (a dim-256 tile's operands need 256 registers a lane)
+template <int D>
+constexpr int kFewThreads = D <= 128 ? 1024 : 512;
+constexpr int kFewTiles = 4;
+constexpr int64_t kFewBytes = 128 << 20;
 constexpr int kSelectThreads = 256;
 constexpr int kSelectSlots = 4096;   // candidates gathered into LDS for the selection
 constexpr int kMaxTopk = 2048;
@@ -57,6 +62,7 @@ constexpr uint32_t kCandidateCapacity = 32768;  // per query
 constexpr int kMaxSegments = 256;
 constexpr uint32_t kSegmentSlots = kCandidateCapacity - kMaxTopk;
 constexpr int64_t kRoundAlign = 2048;
+constexpr int64_t kRoundCandidates = 1 << 17;
 
 // Monotone map of floats to unsigned ints (larger float -> larger int).
 __device__ __forceinline__ uint32_t ordered_bits(float f) {
@@ -76,23 +82,18 @@ __device__ __forceinline__ uint64_t make_key(float score, int64_t doc) {
 }
 
 struct TopkState {
-  uint32_t* counts;    // [Q] best candidates kept (<= topk)
+  uint32_t* counts;    // [Q] best candidates kept (<= topk), and kOverflowed
   float* thr;          // [Q] entry threshold
   uint64_t* cand;      // [Q * capacity] keys
-  uint32_t* segn;      // [Q * kMaxSegments] entries in each segment
-  uint32_t* overflow;  // [1]
+  uint32_t* segn;      // [Q * kMaxSegments] candidates found for each segment
   uint32_t capacity;
   uint32_t seg;        // slots per segment in the current round
+  int first_round;     // counts and thr are not written yet: none kept, -inf
 };
 
-__global__ void topk_reset_kernel(TopkState st, int64_t num_queries) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < num_queries) {
-    st.counts[i] = 0u;
-    st.thr[i] = -INFINITY;
-  }
-  if (i == 0) st.overflow[0] = 0u;
-}
+// In counts: a segment of the query was too small in this round or an earlier
+// one.
+constexpr uint32_t kOverflowed = 0x80000000u;
 
 // Scoring geometry for embedding dimension D.  Each of the 8 waves keeps
 // QT query tiles (32 queries each) as MFMA B operands in registers, so one
@@ -179,7 +180,6 @@ __device__ __forceinline__ void tile_candidates(const TopkState& st, const f32x1
       for (int i = 0; i < 16; ++i) v = j == i ? acc[i] : v;
       const int64_t doc = doc0 + 8 * (j >> 2) + 4 * h + (j & 3);
       if (slot < st.seg) seg[slot] = make_key(v, doc);
-      else atomicOr(st.overflow, 1u);
       ++slot;
     }
   }
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kScoreThreads) void topk_score_kernel(
       b[t][s] = *reinterpret_cast<const bf16x8*>(row + s * 16);
       if (!valid) b[t][s] = bf16x8{};
     }
-    th[t] = st.thr[q_begin + (valid ? ql[t] : 0)];
+    th[t] = st.first_round ? -INFINITY : st.thr[q_begin + (valid ? ql[t] : 0)];
   }
 
   u32x4 dpre[SS::kDocLoads];
@@ -385,7 +385,82 @@ __global__ __launch_bounds__(kScoreThreads) void topk_score_kernel(
     }
   }
   __syncthreads();
-  for (int i = tid; i < q_count; i += kScoreThreads) segn[i * kMaxSegments] = min(slot_count[i], st.seg);
+  for (int i = tid; i < q_count; i += kScoreThreads) segn[i * kMaxSegments] = slot_count[i];
+}
+
+// Scores docs [lo, hi) for few queries: grid.y tiles of 32, of which each wave
+// holds one as B operands.  The waves share out the 64-doc columns of the mask
+// and read their rows straight from memory as A operands, so that nothing is
+// staged and a small corpus has every column in flight at once (topk_score_kernel
+// gives a CU's waves different queries and takes the docs in steps: with 16
+// queries one wave of eight works, 10 us for a step or two).  Rows that no
+// query of the tile passes are not read.  The same products in the same order
+// as topk_score_kernel's.  Latency-bound on small corpora (16 queries, 200,000
+// docs, dim 64: the call 134 -> 55 us with this kernel, two rounds and the
+// overflow flag in host memory), bandwidth-bound on large ones (16 queries, 20M
+// docs, dim 128: 1.34 -> 0.78 ms).
+template <int D>
+__global__ __launch_bounds__(kFewThreads<D>) void topk_score_few_kernel(
+    const uint16_t* __restrict__ emb, const uint16_t* __restrict__ qv,
+    const uint64_t* __restrict__ mask64, int64_t num_columns, int64_t num_queries, int64_t lo,
+    int64_t hi, TopkState st) {
+  constexpr int S = D / 16;
+  __shared__ uint32_t slot_count[kQueryTile];
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, row = lane & 31;
+  const int64_t q0 = static_cast<int64_t>(blockIdx.y) * kQueryTile;
+  const int64_t q = q0 + row;
+  const bool valid = q < num_queries;
+  if (tid < kQueryTile) slot_count[tid] = 0u;
+  __syncthreads();
+  const int64_t columns = (hi + 63) >> 6;
+  const int64_t wave = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(tid >> 6)) * gridDim.x + blockIdx.x;
+  const int64_t waves = static_cast<int64_t>(kFewThreads<D> / 64) * gridDim.x;
+  const uint64_t* mrow = mask64 + (valid ? q : q0) * num_columns;
+  int64_t col = (lo >> 6) + wave;
+  uint64_t next = valid && col < columns ? mrow[col] : 0ull;
+  if (col < columns) {
+    bf16x8 b[S];
+    const uint16_t* src = qv + (valid ? q : q0) * D + h * 8;
+#pragma unroll
+    for (int s = 0; s < S; ++s) b[s] = *reinterpret_cast<const bf16x8*>(src + s * 16);
+    const float th = st.first_round ? -INFINITY : st.thr[valid ? q : q0];
+    for (; col < columns; col += waves) {
+      uint64_t m = next;
+      const int64_t ahead = col + waves;
+      next = valid && ahead < columns ? mrow[ahead] : 0ull;
+      const int64_t left = hi - (col << 6);
+      if (left < 64) m &= ~0ull << (64 - static_cast<int>(left));
+      // docs that some query of the tile passes
+      uint32_t any[2] = {static_cast<uint32_t>(m >> 32), static_cast<uint32_t>(m)};
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+#pragma unroll
+        for (int d = 1; d < 32; d <<= 1) any[x] |= __shfl_xor(any[x], d, 64);
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        if (__builtin_amdgcn_readfirstlane(any[x]) == 0u) continue;
+        const int64_t doc0 = (col << 6) + 32 * x;
+        bf16x8 a[S];
+        if ((any[x] >> (31 - row)) & 1u) {
+          const uint16_t* r = emb + (doc0 + row) * D + h * 8;
+#pragma unroll
+          for (int s = 0; s < S; ++s) a[s] = *reinterpret_cast<const bf16x8*>(r + s * 16);
+        } else {
+#pragma unroll
+          for (int s = 0; s < S; ++s) a[s] = bf16x8{};
+        }
+        f32x16 acc = {};
+#pragma unroll
+        for (int s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], b[s], acc, 0, 0, 0);
+        const uint32_t mx = x == 0 ? static_cast<uint32_t>(m >> 32) : static_cast<uint32_t>(m);
+        if (__ballot(tile_gate(acc, mx, th)) != 0)
+          tile_candidates(st, acc, mx, th, q, slot_count + row, doc0, lane);
+      }
+    }
+  }
+  __syncthreads();
+  if (tid < kQueryTile && q < num_queries) st.segn[q * kMaxSegments + blockIdx.x] = slot_count[tid];
 }
 
 // Descending bitonic sort of the first `size` keys in LDS (a power of two).
@@ -526,16 +601,19 @@ __device__ uint32_t select_best(Key key_at, uint64_t* keys, uint32_t n, uint32_t
 // of the round's nseg segments, gathered in that order.
 __global__ __launch_bounds__(kSelectThreads) void topk_select_kernel(
     TopkState st, int64_t topk, int nseg, int final_round, int64_t* __restrict__ out_ids,
-    float* __restrict__ out_scores) {
+    float* __restrict__ out_scores, uint32_t* __restrict__ overflow) {
   static_assert(kSelectThreads == kMaxSegments, "one thread per segment");
   __shared__ uint64_t keys[kSelectSlots];
   __shared__ uint32_t start[kMaxSegments + 1];  // virtual index of each segment's first entry
   const int64_t q = blockIdx.x;
   uint64_t* cand = st.cand + q * st.capacity;
-  const uint32_t kept = st.counts[q];
+  const uint32_t count = st.first_round ? 0u : st.counts[q];
+  const uint32_t kept = count & ~kOverflowed;
   // Exclusive scan of the segment counts, one thread per segment.
   const int g = threadIdx.x;
-  const uint32_t mine = g < nseg ? min(st.segn[q * kMaxSegments + g], st.seg) : 0u;
+  const uint32_t found = g < nseg ? st.segn[q * kMaxSegments + g] : 0u;
+  const uint32_t mine = min(found, st.seg);
+  const bool over = __syncthreads_or(found > st.seg) != 0 || count > kept;
   start[g + 1] = mine;
   if (g == 0) start[0] = 0u;
   __syncthreads();
@@ -571,6 +649,7 @@ __global__ __launch_bounds__(kSelectThreads) void topk_select_kernel(
     best = select_best(at, keys, n, static_cast<uint32_t>(topk), &sel_min);
   }
   if (final_round) {
+    if (over && threadIdx.x == 0) *overflow = 1u;  // host memory
     int size = 64;
     while (size < static_cast<int>(best)) size <<= 1;
     for (int i = static_cast<int>(best) + threadIdx.x; i < size; i += kSelectThreads) keys[i] = 0ull;
@@ -585,7 +664,7 @@ __global__ __launch_bounds__(kSelectThreads) void topk_select_kernel(
   }
   for (uint32_t i = threadIdx.x; i < best; i += kSelectThreads) cand[i] = keys[i];
   if (threadIdx.x == 0) {
-    st.counts[q] = best;
+    st.counts[q] = best | (over ? kOverflowed : 0u);
     st.thr[q] = best == topk ? from_ordered(static_cast<uint32_t>(sel_min >> 32)) : -INFINITY;
   }
 }
@@ -620,14 +699,41 @@ int launch_score(const uint16_t* emb, const uint16_t* qv, const uint64_t* mask64
   return grid;
 }
 
+// The same for few queries, with topk_score_few_kernel.
+template <int D>
+int launch_score_few(const uint16_t* emb, const uint16_t* qv, const uint64_t* mask64,
+                     int64_t num_columns, int64_t num_queries, int64_t lo, int64_t hi,
+                     TopkState st, bool need_fit, hipStream_t s) {
+  const int64_t columns = ((hi + 63) >> 6) - (lo >> 6);
+  const int64_t groups = std::min<int64_t>(cu_count(), kMaxSegments);
+  const int64_t per_group = (columns + groups - 1) / groups;
+  const int grid = static_cast<int>((columns + per_group - 1) / per_group);
+  const unsigned tiles = static_cast<unsigned>((num_queries + kQueryTile - 1) / kQueryTile);
+  st.seg = kSegmentSlots / static_cast<uint32_t>(grid);
+  if (need_fit && static_cast<int64_t>(st.seg) < per_group * 64)
+    fail("internal: a segment of ", st.seg, " slots cannot hold ", per_group * 64, " docs");
+  hipLaunchKernelGGL(topk_score_few_kernel<D>, dim3(grid, tiles), dim3(kFewThreads<D>), 0, s, emb, qv,
+                     mask64, num_columns, num_queries, lo, hi, st);
+  check_launch("topk_score_few_kernel");
+  return grid;
+}
+
 using ScoreFn = int (*)(const uint16_t*, const uint16_t*, const uint64_t*, int64_t, int64_t,
                         int64_t, int64_t, TopkState, bool, hipStream_t);
 
-ScoreFn score_fn(int64_t dim) {
+// One tile of queries reads every row once; more tiles read the rows again, from
+// the last-level cache while they fit it (64 queries over 400,000 docs of dim
+// 128: 211 us staged, 148 us so; 128 queries: 220 and 184 us).
+bool few_queries(int64_t num_queries, int64_t num_docs, int64_t dim) {
+  const int64_t tiles = (num_queries + kQueryTile - 1) / kQueryTile;
+  return tiles == 1 || (tiles <= kFewTiles && num_docs * dim * 2 <= kFewBytes);
+}
+
+ScoreFn score_fn(int64_t dim, bool few) {
   switch (dim) {
-    case 64: return launch_score<64>;
-    case 128: return launch_score<128>;
-    case 256: return launch_score<256>;
+    case 64: return few ? launch_score_few<64> : launch_score<64>;
+    case 128: return few ? launch_score_few<128> : launch_score<128>;
+    case 256: return few ? launch_score_few<256> : launch_score<256>;
     default: fail("embedding dimension ", dim, " is not supported (64, 128 or 256)");
   }
 }
@@ -651,23 +757,77 @@ void set_lds_limits() {
     throw Error(ST_ERR_HIP, cat("hipFuncSetAttribute failed: ", hipGetErrorString(status)));
 }
 
-// Doc ranges of the rounds: a first round of 8192 docs, then each round
-// eight times everything before it (rounds aligned to bundles), or, in the
-// safe schedule, rounds no larger than the candidate segments can always hold.
-std::vector<int64_t> round_bounds(int64_t num_docs, bool safe) {
+// Doc ranges of the rounds (aligned to bundles): a first round without a
+// threshold, then each round `growth` times everything before it, which leaves
+// about growth x topk candidates per query.  A round takes about 20 us of fixed
+// time and a candidate about 0.4 ns, so growth lies where a round's candidates
+// cost a few rounds (kRoundCandidates over all queries), between 8 (512 queries
+// of 100: 2.9-3.0 ms; x4 and x12 no faster) and half of what the selection
+// holds in LDS (16 queries of 10 over 200,000 docs: two rounds instead of
+// three).  512 queries of 10 over 1M docs: 0.29 ms with x8, 0.72 ms with x204.
+// In the safe schedule no round is larger than the candidate segments can
+// always hold.
+std::vector<int64_t> round_bounds(int64_t num_docs, int64_t num_queries, int64_t topk, bool safe) {
   std::vector<int64_t> b{0};
   int64_t pos = 0;
   // A safe round gives each workgroup at most one segment's worth of docs.
   static_assert(kSegmentSlots % kRoundAlign == 0, "safe rounds stay aligned");
   const int64_t safe_step = kSegmentSlots;
+  const int64_t growth =
+      std::max<int64_t>(8, std::min(kSelectSlots / 2 / topk, kRoundCandidates / (num_queries * topk)));
+  const int64_t first = topk <= 64 ? 2048 : 8192;
   while (pos < num_docs) {
-    int64_t step = safe ? safe_step : (pos == 0 ? 8192 : 8 * pos);
+    int64_t step = safe ? safe_step : (pos == 0 ? first : growth * pos);
     step = (step + kRoundAlign - 1) / kRoundAlign * kRoundAlign;
     pos = std::min(num_docs, pos + step);
     b.push_back(pos);
   }
   return b;
 }
+
+// Words of pinned host memory that the last kernel of a call stores its
+// overflow flag to (a copy of the flag and the wait for it cost more than the
+// small selections themselves).  A call holds one from before its first launch
+// until it has waited for its stream; there are as many as calls ever ran at
+// once.
+class HostFlag {
+ public:
+  HostFlag() {
+    {
+      std::lock_guard<std::mutex> lk(mutex());
+      if (!spare().empty()) {
+        word_ = spare().back();
+        spare().pop_back();
+      }
+    }
+    if (word_ == nullptr) {
+      void* p = nullptr;
+      const hipError_t e = hipHostMalloc(&p, 64, hipHostMallocCoherent | hipHostMallocPortable);
+      if (e != hipSuccess) throw Error(ST_ERR_HIP, cat("hipHostMalloc failed: ", hipGetErrorString(e)));
+      word_ = static_cast<uint32_t*>(p);
+    }
+    __atomic_store_n(word_, 0u, __ATOMIC_RELEASE);
+  }
+  ~HostFlag() {
+    std::lock_guard<std::mutex> lk(mutex());
+    spare().push_back(word_);
+  }
+  HostFlag(const HostFlag&) = delete;
+  HostFlag& operator=(const HostFlag&) = delete;
+  uint32_t* word() const { return word_; }
+  bool set() const { return __atomic_load_n(word_, __ATOMIC_ACQUIRE) != 0u; }
+
+ private:
+  static std::mutex& mutex() {
+    static std::mutex* m = new std::mutex;
+    return *m;
+  }
+  static std::vector<uint32_t*>& spare() {
+    static auto* v = new std::vector<uint32_t*>;
+    return *v;
+  }
+  uint32_t* word_ = nullptr;
+};
 
 }  // namespace
 }  // namespace st
@@ -697,14 +857,14 @@ extern "C" int st_filtered_topk(const int64_t* packed, int64_t num_queries,
     ST_CHECK(reinterpret_cast<uintptr_t>(doc_embeddings) % 16 == 0 &&
                  reinterpret_cast<uintptr_t>(query_embeddings) % 16 == 0,
              "embeddings must be 16-byte aligned");
-    const ScoreFn score = score_fn(dim);
+    const bool few = few_queries(num_queries, num_docs, dim);
+    const ScoreFn score = score_fn(dim, few);
     set_lds_limits();
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     TopkState state;
     state.counts = reinterpret_cast<uint32_t*>(ws);
     state.thr = reinterpret_cast<float*>(ws + 4 * num_queries);
-    state.overflow = reinterpret_cast<uint32_t*>(ws + 8 * num_queries);
     state.cand = reinterpret_cast<uint64_t*>(ws + ((8 * num_queries + 4 + 255) / 256) * 256);
     state.capacity = kCandidateCapacity;
     state.segn = reinterpret_cast<uint32_t*>(state.cand + num_queries * static_cast<int64_t>(kCandidateCapacity));
@@ -713,36 +873,34 @@ extern "C" int st_filtered_topk(const int64_t* packed, int64_t num_queries,
     const uint16_t* qv = static_cast<const uint16_t*>(query_embeddings);
     const uint64_t* m64 = reinterpret_cast<const uint64_t*>(packed);
     const unsigned qgrid = static_cast<unsigned>(num_queries);
+    HostFlag overflow;
 
     for (int attempt = 0; attempt < 2; ++attempt) {
       const bool safe = attempt == 1;
-      hipLaunchKernelGGL(topk_reset_kernel, dim3(static_cast<unsigned>((num_queries + 255) / 256)),
-                         dim3(256), 0, s, state, num_queries);
-      check_launch("topk_reset_kernel");
-      const std::vector<int64_t> bounds = round_bounds(num_docs, safe);
+      const std::vector<int64_t> bounds = round_bounds(num_docs, num_queries, topk, safe);
       for (size_t r = 0; r + 1 < bounds.size(); ++r) {
+        state.first_round = r == 0 ? 1 : 0;
         const int nseg = score(emb, qv, m64, num_columns, num_queries, bounds[r], bounds[r + 1],
                                state, safe, s);
         TopkState sel = state;
         sel.seg = kSegmentSlots / static_cast<uint32_t>(nseg);
         const bool last = r + 2 == bounds.size();
         hipLaunchKernelGGL(topk_select_kernel, dim3(qgrid), dim3(kSelectThreads), 0, s, sel,
-                           topk, nseg, last ? 1 : 0, out_ids, out_scores);
+                           topk, nseg, last ? 1 : 0, out_ids, out_scores, overflow.word());
         check_launch("topk_select_kernel");
       }
       if (bounds.size() == 1) {  // no docs: every output is padding
+        state.first_round = 1;
         hipLaunchKernelGGL(topk_select_kernel, dim3(qgrid), dim3(kSelectThreads), 0, s, state,
-                           topk, 0, 1, out_ids, out_scores);
+                           topk, 0, 1, out_ids, out_scores, overflow.word());
         check_launch("topk_select_kernel");
         return;
       }
       if (safe) return;  // rounds of this schedule cannot overflow
-      uint32_t overflow = 0;
-      hipError_t e = hipMemcpyAsync(&overflow, state.overflow, 4, hipMemcpyDeviceToHost, s);
-      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      const hipError_t e = hipStreamSynchronize(s);
       if (e != hipSuccess)
-        throw Error(ST_ERR_HIP, cat("reading the overflow flag failed: ", hipGetErrorString(e)));
-      if (!overflow) return;
+        throw Error(ST_ERR_HIP, cat("waiting for the selection failed: ", hipGetErrorString(e)));
+      if (!overflow.set()) return;
     }
   });
 }

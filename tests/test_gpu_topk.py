@@ -123,6 +123,27 @@ def test_topk_ties_overflow_and_safe_rounds(dim):
     assert (sc[0] == dim).all() and (ids[1] == -1).all() and np.isneginf(sc[1]).all()
 
 
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("n,topk", [(31, 3), (64, 1), (70_001, 10), (40_000, 65), (140_000, 2048)])
+def test_topk_few_queries_as_in_a_batch(dim, n, topk):
+    """A few queries (their tiles of 32 read the docs straight from memory: 1,
+    32, 33 and 128 queries) against the same queries in a batch of 150 (staged
+    steps): the same products in the same order, so the same bits; the batch
+    against the oracle."""
+    rng = np.random.default_rng(dim + n + topk)
+    emb_bf, qv_bf, emb32, qv32, packed = _random_case(rng, n, dim, 150, 0.3)
+    packed[3] = 0                                     # nothing passes
+    packed[5] &= (rng.random(packed.shape[1]) < 0.02).astype(np.int64) * -1  # few columns hold a doc
+    H.note(f"[topk few] dim={dim} n={n} topk={topk}")
+    ids, sc = _gpu_topk(packed, emb_bf, qv_bf, n, topk)
+    _check(ids[:8], sc[:8], emb32, qv32[:8], packed[:8], n, topk)
+    _check(ids[-2:], sc[-2:], emb32, qv32[-2:], packed[-2:], n, topk)
+    for q in (1, 32, 33, 128):
+        few_ids, few_sc = _gpu_topk(packed[:q], emb_bf, qv_bf[:q], n, topk)
+        np.testing.assert_array_equal(few_ids, ids[:q])
+        np.testing.assert_array_equal(few_sc.view(np.uint32), sc[:q].view(np.uint32))
+
+
 def test_topk_ties_at_the_boundary_go_to_lower_ids():
     """300 docs share one embedding row whose score falls near rank 60 of the
     top 100, so the boundary of the top 100 cuts through the group: equal
