@@ -162,6 +162,14 @@ int st_search_plan_bind_widths(st_search_plan* plan,
  * st_search_plan_bind_widths. */
 int st_search_plan_prepare_device_binding(st_search_plan* plan,
                                           int64_t num_bundles);
+
+/* Whether a search of an index of bloom_index_numel words in num_bundles
+ * bundles is expected to be faster with the plan bound to the bundle widths
+ * (packed_out: 1 for the packed output of st_bloom_index_search_batch, 0 for its
+ * bool mask and for the counts of st_bloom_index_search_batch_counts).  The
+ * results are the same either way. */
+int st_search_plan_wants_binding(const st_search_plan* plan, int64_t bloom_index_numel,
+                                 int64_t num_bundles, int packed_out);
 int64_t st_search_plan_device_bytes(const st_search_plan* plan);
 /* Optional: the search calls with this plan copy the blob into
  * plan_blob_device themselves, in their first kernel, from `pinned_host` --

@@ -74,6 +74,10 @@ namespace {
 // The host-side equivalent is st_search_plan_bind_widths (search_plan.cpp).
 
 constexpr int kBindThreads = 1024;
+// Limits of the searches that go unbound (st_search_plan_wants_binding).
+constexpr int64_t kDirectReads = 32;
+constexpr int64_t kUnboundWideReads = 240;
+constexpr int64_t kUnboundBoolQueries = 64;
 constexpr int kBindGrid = 256;     // workgroups of the binding kernel
 // Distinct widths the census tracks.  An index with more gets no slots at
 // all (every bundle resolves its positions itself): whether the table
@@ -490,6 +494,18 @@ static_assert(kOutPacked == kGenericPacked && kOutBool == kGenericBool &&
                   kOutCounts == kGenericCounts,
               "one output-mode numbering for the batch and generic kernels");
 
+// Rows of a bundle that the plan's terms name (each batch's distinct terms).
+int64_t row_reads(const st_search_plan* plan) {
+  int64_t terms = 0;
+  for (const SearchBatch& bt : plan->batches) terms += bt.num_terms;
+  return terms * std::max(plan->k_eff, 1);
+}
+
+// Whether the mean bundle is wider than the LDS tile.
+bool wide_rows(int64_t bloom_index_numel, int64_t num_bundles) {
+  return bloom_index_numel / kColumnsPerBundle > num_bundles * kSearchTileRows;
+}
+
 // Validates the arguments and launches the search kernel once per batch.
 void launch_search(const int64_t* bloom_index, int64_t bloom_index_numel,
                    const int64_t* bundle_b_offsets, int64_t num_bundles,
@@ -501,8 +517,13 @@ void launch_search(const int64_t* bloom_index, int64_t bloom_index_numel,
   ST_CHECK(plan->bound_bundles < 0 || plan->bound_bundles == num_bundles,
            "plan was bound to ", plan->bound_bundles, " bundles, the index has ",
            num_bundles);
+  // An unbound search of few wide bundles splits each by program over the
+  // workgroups that have no bundle (the kernel's last round): 16 trees over 49
+  // bundles of 1,760 rows 50 -> 34 us.  Narrow bundles have a tile to stage in
+  // each workgroup and gain nothing.
+  const bool split = plan->bound_bundles < 0 && wide_rows(bloom_index_numel, num_bundles);
   const int grid = static_cast<int>(
-      std::min<int64_t>(num_bundles, static_cast<int64_t>(device_cu_count())));
+      split ? device_cu_count() : std::min<int64_t>(num_bundles, device_cu_count()));
   const char* blob = static_cast<const char*>(plan_blob_device);
   const bool bound = plan->bound_bundles >= 0;
   auto at = [&](uint64_t off) { return reinterpret_cast<const uint32_t*>(blob + off); };
@@ -615,6 +636,10 @@ void launch_search(const int64_t* bloom_index, int64_t bloom_index_numel,
     const bool quad = bound && bt.stream_words != 0 &&
                       bt.stream_words <= kQuadStreamMaxWords &&
                       stream_block_records(kk) >= 4;
+    // Few rows of each bundle are named: they are read from memory instead of
+    // the whole tile (one query of four terms over 8M docs of 450-row bundles:
+    // 61 us, 92 us with tiles; four queries: 113 and 111 us).
+    const bool direct = !bound && row_reads(plan) <= kDirectReads;
     KernelFn fn = select_kernel(plan->k_eff, mode, quad);
     hipLaunchKernelGGL(
         fn, dim3(grid), dim3(kSearchThreads), 0, stream, bloom_index, bloom_index_numel,
@@ -630,7 +655,7 @@ void launch_search(const int64_t* bloom_index, int64_t bloom_index_numel,
         bound ? at(bt.off_stream_skip) : nullptr, bound ? bt.stream_off : 0u,
         bound ? bt.stream_words : 0u, bound ? bt.stream_masks : 0u, bt.num_terms,
         static_cast<int32_t>(plan->hash_k),
-        num_bundles * 32, out, counts, num_docs, wide_flag,
+        num_bundles * 32, out, counts, num_docs, direct ? kDirectRows : wide_flag,
         plan->device_bind ? at(plan->off_num_slots) : nullptr,
         carry_wide ? at(plan->off_wide) : nullptr,
         carry_wide ? at(plan->off_bundle_order) : nullptr,
@@ -659,6 +684,26 @@ void compact_scan_counts(int64_t* counts, int64_t num_queries, int64_t nch,
 void compact_zero_offsets(int64_t* row_offsets, int64_t n, hipStream_t s);
 
 }  // namespace st
+
+// Binding costs two launches' work ahead of the search (~10 us and more host
+// time) and pays where many bundles share a width, or where it lets wide
+// bundles be streamed.  Measured with and without, us: 500,000 docs of 450-row
+// bundles, 16 queries 31 / 25, 1M docs 64 queries packed 43 / 38, 2M docs 52 /
+// 57; bool output of 256 queries over 1M docs 102 / 152; wide bundles (1,760
+// rows) packed, 4 trees over 12M docs 677 / 531, 16 trees 837 / 1,022, 256
+// trees over 500,000 docs 350 / 305; wide bundles with bool output (never
+// streamed), 64 trees over 2M docs 499 / 324.
+extern "C" int st_search_plan_wants_binding(const st_search_plan* plan, int64_t bloom_index_numel,
+                                            int64_t num_bundles, int packed_out) {
+  using namespace st;
+  if (plan == nullptr || num_bundles <= 0) return 0;
+  const int64_t cus = device_cu_count();
+  const int64_t reads = row_reads(plan);
+  if (wide_rows(bloom_index_numel, num_bundles))
+    return packed_out != 0 && num_bundles > cus && reads > kUnboundWideReads;
+  if (reads <= kDirectReads) return 0;
+  return num_bundles > 2 * cus || (packed_out == 0 && plan->num_queries > kUnboundBoolQueries);
+}
 
 extern "C" int st_search_plan_upload_source(st_search_plan* plan, const void* pinned_host) {
   using namespace st;

@@ -119,6 +119,9 @@ struct BundleMeta {
 // The bundles of the grid's last, partial round are split among up to this
 // many workgroups each, by program.
 constexpr int kTailParts = 4;
+// wide_skip of a launch of an unbound plan whose few terms' rows are read
+// straight from memory.
+constexpr uint32_t kDirectRows = 4;
 
 // Cycles a program or round counter through the parts of a split visit.
 struct PartFilter {
@@ -1033,12 +1036,14 @@ __global__ __launch_bounds__(kSearchThreads) void bloom_search_kernel(
       sp[i] = c < chunks ? src[c] : u32x4{0, 0, 0, 0};
     }
   };
+  // Rows read straight from memory, no tile (kDirectRows).
+  const bool direct = !kQuad && (wide_skip & kDirectRows) != 0;
   u32x4 pre[kPrefetch];
   u32x4 spre[kQuad ? kStreamPrefetch : 1];
   const BundleMeta none{-1, 0, 0, kNoWidthSlot, 0, 1};
   BundleMeta cur = search_phase ? visit(0) : none, nxt = search_phase ? visit(1) : none;
   if (cur.bundle >= 0) {
-    prefetch_tile(a, cur.start, cur.b, pre);
+    if (!direct) prefetch_tile(a, cur.start, cur.b, pre);
     if (quad_bundle(cur)) prefetch_stream(cur, spre);
   }
 
@@ -1060,7 +1065,7 @@ __global__ __launch_bounds__(kSearchThreads) void bloom_search_kernel(
     const PartFilter pf{cur.part, cur.parts, 0u};
     const int64_t start = cur.start, b = cur.b;
     const uint32_t slot = cur.slot;
-    const bool staged = b <= kSearchTileRows;
+    const bool staged = b <= kSearchTileRows && !direct;
 
     const bool quad_here = quad_bundle(cur);
     // the wide-bundle kernel evaluates the literal stream of this bundle
@@ -1096,7 +1101,7 @@ __global__ __launch_bounds__(kSearchThreads) void bloom_search_kernel(
     // another slot's is in LDS.
     const bool has_next = nxt.bundle >= 0;
     if (has_next) {
-      prefetch_tile(a, nxt.start, nxt.b, pre);
+      if (!direct) prefetch_tile(a, nxt.start, nxt.b, pre);
       if (quad_bundle(nxt) && nxt.slot != staged_slot) prefetch_stream(nxt, spre);
     }
     if (!skip && slot == kNoWidthSlot && b != prev_b) {

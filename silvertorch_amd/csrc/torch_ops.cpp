@@ -276,7 +276,7 @@ struct PreparedSearch {
 
 void prepare_search(PreparedSearch& ps, const Tensor& bloom_index_in,
                     const Tensor& bundle_b_offsets_in, const Tensor& plans_data,
-                    const Tensor& plans_offsets, int64_t k, int64_t hash_k) {
+                    const Tensor& plans_offsets, int64_t k, int64_t hash_k, bool packed_out) {
   TORCH_CHECK(bloom_index_in.is_cuda(), "bloom_index must be a GPU tensor");
   TORCH_CHECK(bloom_index_in.dim() == 1, "bloom_index must be 1-D");
   TORCH_CHECK(bloom_index_in.scalar_type() == at::kLong, "bloom_index must be int64");
@@ -305,8 +305,10 @@ void prepare_search(PreparedSearch& ps, const Tensor& bloom_index_in,
   ps.nb = ps.bbo.numel() - 1;
   if (ps.Q == 0 || ps.nb == 0) return;
   // The search call binds the programs to the bundle widths on the device
-  // (no copy of the bundle offsets to the host, no synchronisation).
-  check_st(st_search_plan_prepare_device_binding(ps.plan.p, ps.nb), "bloom_index_search_batch");
+  // (no copy of the bundle offsets to the host, no synchronisation), where
+  // that pays.
+  if (st_search_plan_wants_binding(ps.plan.p, ps.index.numel(), ps.nb, packed_out ? 1 : 0))
+    check_st(st_search_plan_prepare_device_binding(ps.plan.p, ps.nb), "bloom_index_search_batch");
   // The plan bytes go to pinned memory of torch's host allocator, and the
   // search call's first kernel copies them to the device on the caller's
   // stream (no copy-engine hand-off between the previous call's kernels and
@@ -348,7 +350,7 @@ Tensor search_gpu(const Tensor& bloom_index_in, const Tensor& bundle_b_offsets_i
   c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(bloom_index_in.device());
   PreparedSearch ps;
   prepare_search(ps, bloom_index_in, bundle_b_offsets_in, plans_data, plans_offsets, k,
-                 hash_k);
+                 hash_k, !return_bool_mask);
   const auto dev = ps.index.device();
   const int64_t C = ps.nb * ST_COLUMNS_PER_BUNDLE;
   Tensor out = return_bool_mask
@@ -719,7 +721,8 @@ std::tuple<Tensor, Tensor> search_ids_gpu(const Tensor& bloom_index,
                 "int32 ids cannot hold doc ids up to ", num_docs, "; pass int64_ids=True");
   }
   PreparedSearch ps;
-  prepare_search(ps, bloom_index, bundle_b_offsets, plans_data, plans_offsets, k, hash_k);
+  prepare_search(ps, bloom_index, bundle_b_offsets, plans_data, plans_offsets, k, hash_k,
+                 /*packed_out=*/false);
   const auto dev = ps.index.device();
   const int64_t C = ps.nb * ST_COLUMNS_PER_BUNDLE;
   auto opts = at::TensorOptions().device(dev);

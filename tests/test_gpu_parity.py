@@ -198,6 +198,34 @@ def test_build_tile_shapes_vs_oracle(widest, docs, F):
     assert int(np.diff(bbo).max()) >= widest
 
 
+@pytest.mark.parametrize("docs,bm", [(9000, 5.0), (9000, 60.0), (9000, 200.0), (1_050_000, 5.0), (530_000, 60.0)])
+@pytest.mark.parametrize("num_queries", [1, 9, 64, 65, 130])
+def test_search_op_with_and_without_binding(docs, bm, num_queries):
+    """The operator's choice of a bound or an unbound plan (and of rows read
+    without a tile for a term or two) at both sides of its limits: 9,000 docs
+    are 5 bundles, 1,050,000 are 513; b is ~50, ~600 (wider than the tile) or
+    ~2,000 rows; packed, bool and counted outputs against the oracle."""
+    rng = np.random.default_rng(docs + num_queries)
+    ids, offs, vals = _random_corpus(rng, docs, 2, 0, 3, 40)
+    index, bbo = O.bloom_build(ids, offs, vals, bm, 2)
+    term = lambda: ("NOT " if rng.random() < 0.2 else "") + f"{int(rng.choice(ids))}:{int(rng.integers(0, 45))}"
+    queries = [term() if i % 3 == 0 else f"{term()} AND ({term()} OR {term()})" for i in range(num_queries)]
+    pd, po = _plans(queries, 5, 5)
+    want = O.search_packed(index, bbo, pd, po, 2, 5)
+    H.note(f"[op binding] docs={docs} bm={bm} queries={num_queries}")
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (index, bbo)]
+    plans = [torch.from_numpy(np.ascontiguousarray(a)) for a in (pd, po)]
+    got = torch.ops.st.bloom_index_search_batch(*t, *plans, 2, 5, False).cpu().numpy()
+    np.testing.assert_array_equal(got, want)
+    if docs * num_queries < 40_000_000:
+        mask = torch.ops.st.bloom_index_search_batch(*t, *plans, 2, 5, True).cpu().numpy()
+        np.testing.assert_array_equal(mask, O.unpack_bool(want))
+    _, row_offsets = torch.ops.st.bloom_index_search_batch_ids(*t, *plans, 2, 5, docs)
+    bits = np.bitwise_count(want.view(np.uint64)[:, :docs // 64]).sum(1, dtype=np.int64)
+    tail = want.view(np.uint64)[:, docs // 64] >> np.uint64(64 - docs % 64) if docs % 64 else np.zeros(1, np.uint64)
+    np.testing.assert_array_equal(row_offsets.cpu().numpy()[1:], np.cumsum(bits + np.bitwise_count(tail)))
+
+
 def test_many_terms_split_into_passes():
     """More distinct terms than one LDS position area holds -> several passes."""
     rng = np.random.default_rng(77)
