@@ -48,27 +48,78 @@ __device__ __forceinline__ Column column_of(const int64_t* bbo, int64_t col) {
 template <int K>
 __device__ __forceinline__ uint64_t eval_term_word(const EvalArgs& a, const Column& c,
                                                    const ST_EVAL_CONST uint64_t* h) {
+  int16_t found[K];
+  int cnt = 0;
+  uint64_t r = ~0ull;
+  for (int p = 0; p < a.hash_k && cnt < K; ++p) {
+    const int16_t bp = static_cast<int16_t>(fast_mod(h[p], c.fm));
+    bool dup = false;
+#pragma unroll
+    for (int j = 0; j < K; ++j) dup |= (j < cnt) && (found[j] == bp);
+    if (dup) continue;
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+      if (j == cnt) found[j] = bp;
+    ++cnt;
+    const int64_t w = (c.start + bp) * kColumnsPerBundle + c.cib;
+    r &= (w >= 0 && w < a.index_numel) ? static_cast<uint64_t>(a.index[w]) : 0ull;
+  }
+  return r;
+}
+
+// Terms whose rows are read together (kTermsAhead x K words in flight a lane).
+template <int K>
+constexpr int kTermsAhead = K <= 5 ? 4 : 2;
+
+// out[u] = the word of the u-th of n terms (0 < n <= kTermsAhead; the rest are
+// the last's), hashes_of(u) its hashes.  The rows are scattered over the
+// index, so each read is a miss, and what bounds an item is how many of them
+// wait for each other: the first K positions of every term are formed without
+// a branch and their rows read back to back; only a term whose first K positions
+// collide (about K^2 / 2b of them), or with a row outside the index, is evaluated
+// position by position.  K = min(k, hash_k): there are K hashes.
+template <int K, typename HashesOf>
+__device__ __forceinline__ void eval_term_words(const EvalArgs& a, const Column& c, uint32_t n, HashesOf hashes_of,
+                                                uint64_t (&out)[kTermsAhead<K>]) {
+  constexpr int A = kTermsAhead<K>;
   if constexpr (K == 0) {
-    return ~0ull;
+#pragma unroll
+    for (int u = 0; u < A; ++u) out[u] = ~0ull;
   } else {
-    if (c.b <= 0) return 0;
-    int16_t found[K];
-    int cnt = 0;
-    uint64_t r = ~0ull;
-    for (int p = 0; p < a.hash_k && cnt < K; ++p) {
-      const int16_t bp = static_cast<int16_t>(fast_mod(h[p], c.fm));
-      bool dup = false;
 #pragma unroll
-      for (int j = 0; j < K; ++j) dup |= (j < cnt) && (found[j] == bp);
-      if (dup) continue;
+    for (int u = 0; u < A; ++u) out[u] = 0;
+    if (c.b <= 0 || a.index_numel <= 0) return;
+    uint64_t w[A][K];
+    uint32_t again = 0;  // terms to evaluate position by position
 #pragma unroll
-      for (int j = 0; j < K; ++j)
-        if (j == cnt) found[j] = bp;
-      ++cnt;
-      const int64_t w = (c.start + bp) * kColumnsPerBundle + c.cib;
-      r &= (w >= 0 && w < a.index_numel) ? static_cast<uint64_t>(a.index[w]) : 0ull;
+    for (int u = 0; u < A; ++u) {
+      const ST_EVAL_CONST uint64_t* h = hashes_of(u < n ? u : n - 1);
+      int16_t found[K];
+      bool plain = true;
+#pragma unroll
+      for (int j = 0; j < K; ++j) found[j] = static_cast<int16_t>(fast_mod(h[j], c.fm));
+#pragma unroll
+      for (int j = 0; j < K; ++j) {
+#pragma unroll
+        for (int i = 0; i < j; ++i) plain &= found[i] != found[j];
+        const int64_t at = (c.start + found[j]) * kColumnsPerBundle + c.cib;
+        const bool inside = at >= 0 && at < a.index_numel;
+        plain &= inside;
+        w[u][j] = static_cast<uint64_t>(a.index[inside ? at : 0]);
+      }
+      again |= plain ? 0u : 1u << u;
     }
-    return r;
+#pragma unroll
+    for (int u = 0; u < A; ++u) {
+      out[u] = w[u][0];
+#pragma unroll
+      for (int j = 1; j < K; ++j) out[u] &= w[u][j];
+    }
+    if (again != 0) {
+#pragma unroll
+      for (int u = 0; u < A; ++u)
+        if ((again >> u) & 1u) out[u] = eval_term_word<K>(a, c, hashes_of(u < n ? u : n - 1));
+    }
   }
 }
 
@@ -89,15 +140,22 @@ __device__ uint64_t eval_program(const EvalArgs& a, const Column& c,
   auto term_hashes = [&](uint32_t ref) {
     return hashes + static_cast<uint64_t>(ref / a.pos_bytes) * a.hash_k;
   };
+  constexpr uint32_t A = kTermsAhead<K>;
+  uint64_t words[A];
   if (hdr & kFlatForm) {  // OR of AND-groups: [term ref, negate, group, 0]
     const ST_EVAL_CONST uint32_t* lit = prog + kProgHeaderWords;
     uint64_t res = 0, acc = 0;
-    for (uint32_t j = 0; j < T; ++j, lit += kFlatLiteralWords) {
-      const uint64_t w = eval_term_word<K>(a, c, term_hashes(lit[0]));
-      const uint64_t neg = lit[1] ? ~0ull : 0ull;
-      const uint64_t grp = lit[2] ? ~0ull : 0ull;
-      res |= acc & grp;
-      acc = (acc | grp) & (w ^ neg);
+    for (uint32_t j = 0; j < T; j += A, lit += A * kFlatLiteralWords) {
+      const uint32_t n = T - j < A ? T - j : A;
+      eval_term_words<K>(a, c, n, [&](uint32_t u) { return term_hashes(lit[u * kFlatLiteralWords]); }, words);
+#pragma unroll
+      for (uint32_t u = 0; u < A; ++u) {
+        if (u >= n) break;
+        const uint64_t neg = lit[u * kFlatLiteralWords + 1] ? ~0ull : 0ull;
+        const uint64_t grp = lit[u * kFlatLiteralWords + 2] ? ~0ull : 0ull;
+        res |= acc & grp;
+        acc = (acc | grp) & (words[u] ^ neg);
+      }
     }
     res |= acc;
     return (hdr & kFlatComplement) ? ~res : res;
@@ -113,7 +171,15 @@ __device__ uint64_t eval_program(const EvalArgs& a, const Column& c,
     const uint32_t op = ops[i];
     const uint32_t code = op & 7u;
     if (code == kInsTerm) {
-      acc = eval_combine(op, acc, eval_term_word<K>(a, c, term_hashes(tref[t++])));
+      if (t % A == 0) {
+        const uint32_t n = T - t < A ? T - t : A;
+        eval_term_words<K>(a, c, n, [&](uint32_t u) { return term_hashes(tref[t + u]); }, words);
+      }
+      uint64_t word = words[0];
+#pragma unroll
+      for (uint32_t u = 1; u < A; ++u) word = t % A == u ? words[u] : word;
+      ++t;
+      acc = eval_combine(op, acc, word);
     } else if (code == kInsConst) {
       acc = eval_combine(op, acc, ~0ull);
     } else if (code == kInsPush) {

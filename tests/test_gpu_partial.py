@@ -110,6 +110,44 @@ def test_partial_random_vs_oracle(seed):
             np.testing.assert_array_equal(g, w)
 
 
+@pytest.mark.parametrize("k,hk", [(1, 1), (3, 3), (5, 7), (6, 7), (10, 10), (10, 12)])
+@pytest.mark.parametrize("bm", [1.1, 40.0])
+def test_partial_terms_read_together(k, hk, bm):
+    """Runs and trees of 1-9 terms (rows are read for four terms at a time, for
+    two above k = 5: whole groups and remainders), in bundles so narrow that
+    first positions collide and in wide ones, a first bundle without rows, and
+    the same plans on an index cut short (rows outside it read as zero)."""
+    rng = np.random.default_rng(100 * k + hk)
+    n = 7000
+    cnt = rng.integers(0, 4, (n, 1)) * (np.arange(n) >= 2048)[:, None]
+    offs = np.concatenate([[0], np.cumsum(cnt.reshape(-1))]).astype(np.int64)
+    vals = rng.integers(0, 12, int(offs[-1])).astype(np.int64)
+    index, bbo = H.build(np.array([1], dtype=np.int32), offs, vals, bm, k)
+    assert bbo[1] == 0 and bbo[2] > 0
+    queries = []
+    for t in range(1, 10):
+        terms = [("NOT " if rng.random() < 0.2 else "") + f"1:{int(rng.integers(0, 14))}" for _ in range(t)]
+        queries += [" AND ".join(terms), " OR ".join(terms)]
+        tree = terms[0]
+        for i, term in enumerate(terms[1:]):
+            tree = f"({tree}) {'AND' if i % 2 else 'OR'} {term}" if i % 3 else f"{term} OR NOT ({tree})"
+        queries.append(tree)
+    _, data, po = P.parse_batch(queries, hk)
+    pd, po = np.frombuffer(data, dtype=np.int8).copy(), np.array(po, dtype=np.int64)
+    co = np.tile(np.array([[0, 2000, 4096]], dtype=np.int64), (len(queries), 1))
+    cl = np.tile(np.array([[300, 2500, 2900]], dtype=np.int64), (len(queries), 1))
+    H.note(f"[partial together] k={k} hash_k={hk} bm={bm} widths={np.diff(bbo)}")
+    for part in (index, index[:index.size // 2 - 5]):
+        got = _partial("cuda", part, bbo, pd, po, co, cl, k, hk)
+        if part is index:
+            for g, w in zip(got, O.partial_response(index, bbo, pd, po, k, hk, co, cl)):
+                np.testing.assert_array_equal(g, w)
+        else:  # the words past the cut as zeros
+            padded = np.zeros_like(index)
+            padded[:part.size] = part
+            np.testing.assert_array_equal(got[2], O.partial_response(padded, bbo, pd, po, k, hk, co, cl)[2])
+
+
 def test_partial_errors():
     c = G.partial_case("varied_plan_index")
     k, hk = (int(v) for v in c["params"])
