@@ -26,6 +26,7 @@ SIGNATURES = {
     "st_search_plan_create": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, ctypes.POINTER(_vp)]),
     "st_search_plan_bind_widths": (ctypes.c_int, [_vp, _vp, _i64]),
     "st_search_plan_prepare_device_binding": (ctypes.c_int, [_vp, _i64]),
+    "st_search_plan_wants_binding": (ctypes.c_int, [_vp, _i64, _i64, ctypes.c_int]),
     "st_search_plan_device_bytes": (_i64, [_vp]),
     "st_search_plan_upload_source": (ctypes.c_int, [_vp, _vp]),
     "st_search_plan_upload_signal": (ctypes.c_int, [_vp, _vp, ctypes.c_uint64]),
