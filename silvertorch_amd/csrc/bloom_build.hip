@@ -446,7 +446,7 @@ __device__ __forceinline__ void for_each_value(const ScatterArgs& a, const int64
 // meet in its L2.  Parts rather than whole bundles: two tiles fit a CU, so one
 // workgroup hashes while the other clears, loads offsets or stores, and a
 // small corpus (49 bundles at 100,000 docs) still fills the chip.
-// Bound by VALU issue: 236 wave instructions per 64 values at k = 3, one per 4.3
+// Bound by VALU issue: 242 wave instructions per 64 values at k = 3, one per 4.3
 // cycles (nearly every instruction of the hash, 32-bit multiplies and
 // v_mad_u64_u32 included, takes 4).  100M docs x 4 features, 1.8e9 values, 470
 // rows: 12.0 ms; 17.0 ms with a whole bundle per workgroup (one a CU), the

@@ -76,11 +76,6 @@ ST_HD uint64_t murmur_pair(uint64_t x, uint64_t y, uint64_t seed) {
   return murmur_finish(murmur_mix_x(x), murmur_mix_y(y), seed);
 }
 
-// murmur_finish for one key under many small seeds: the seed enters the
-// rotations only through seed ^ mx and seed ^ my, and for seed < 2^27
-// rotl(seed ^ m, r) = rotl(m, r) ^ (seed << r) (r = 27, 31), so the
-// rotations of mx and my are taken once per key (rx = rotl(mx, 27),
-// ry = rotl(my, 31)).  Equal to murmur_finish(mx, my, seed) for those seeds.
 // 5 h: on the device one shift-and-add (the compiler's multiplies by 5 take two
 // and two moves).
 ST_HD uint64_t times5(uint64_t h) {
@@ -92,6 +87,12 @@ ST_HD uint64_t times5(uint64_t h) {
   return h * 5;
 #endif
 }
+
+// murmur_finish for one key under many small seeds: the seed enters the
+// rotations only through seed ^ mx and seed ^ my, and for seed < 2^27
+// rotl(seed ^ m, r) = rotl(m, r) ^ (seed << r) (r = 27, 31), so the
+// rotations of mx and my are taken once per key (rx = rotl(mx, 27),
+// ry = rotl(my, 31)).  Equal to murmur_finish(mx, my, seed) for those seeds.
 ST_HD uint64_t murmur_finish_rot(uint64_t rx, uint64_t ry, uint64_t seed) {
   uint64_t h1 = times5(rx ^ (seed << 27)) + (seed * 5 + 0x52dce729ULL);
   uint64_t h2 = times5((ry ^ (seed << 31)) + h1) + 0x38495ab5ULL;
