@@ -67,17 +67,63 @@ __device__ __forceinline__ uint64_t eval_term_word(const EvalArgs& a, const Colu
   return r;
 }
 
-// Terms whose rows are read together (kTermsAhead x K words in flight a lane).
+// Terms whose rows are read together at most (kTermsAhead x K words in flight a
+// lane).  Two at k = 4 and 5 keep 8 waves a SIMD (five or six with four terms)
+// and measured the same or faster; at k = 3 four cost one wave of eight and
+// gain 10% on trees.
 template <int K>
-constexpr int kTermsAhead = K <= 5 ? 4 : 2;
+constexpr int kTermsAhead = K <= 3 ? 4 : 2;
 
-// out[u] = the word of the u-th of n terms (0 < n <= kTermsAhead; the rest are
-// the last's), hashes_of(u) its hashes.  The rows are scattered over the
-// index, so each read is a miss, and what bounds an item is how many of them
-// wait for each other: the first K positions of every term are formed without
-// a branch and their rows read back to back; only a term whose first K positions
-// collide (about K^2 / 2b of them), or with a row outside the index, is evaluated
-// position by position.  K = min(k, hash_k): there are K hashes.
+// out[u] = the word of the u-th of N terms, hashes_of(u) its hashes.  The rows
+// are scattered over the index, so each read is a miss, and what bounds an item
+// is how many of them wait for each other: the first K positions of every term
+// are formed without a branch and their rows read back to back; only a term
+// whose first K positions collide (about K^2 / 2b of them), or with a row
+// outside the index, is evaluated position by position.  K = min(k, hash_k):
+// there are K hashes.
+template <int K, int N, typename HashesOf>
+__device__ __forceinline__ void eval_term_group(const EvalArgs& a, const Column& c, HashesOf hashes_of,
+                                                uint64_t* out) {
+  uint64_t w[N][K];
+  uint32_t again = 0;  // terms to evaluate position by position
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const ST_EVAL_CONST uint64_t* h = hashes_of(u);
+    int16_t found[K];
+    bool plain = true;
+#pragma unroll
+    for (int j = 0; j < K; ++j) found[j] = static_cast<int16_t>(fast_mod(h[j], c.fm));
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+#pragma unroll
+      for (int i = 0; i < j; ++i) plain &= found[i] != found[j];
+      const int64_t at = (c.start + found[j]) * kColumnsPerBundle + c.cib;
+      const bool inside = at >= 0 && at < a.index_numel;
+      plain &= inside;
+      w[u][j] = static_cast<uint64_t>(a.index[inside ? at : 0]);
+    }
+    again |= plain ? 0u : 1u << u;
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    out[u] = w[u][0];
+#pragma unroll
+    for (int j = 1; j < K; ++j) out[u] &= w[u][j];
+  }
+  if (again != 0) {
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if ((again >> u) & 1u) out[u] = eval_term_word<K>(a, c, hashes_of(u));
+  }
+}
+
+// out[u] = the word of the u-th of n terms (0 < n <= kTermsAhead, uniform over
+// the wave).  A program's last group is as large as what is left of it: with
+// many small clusters the work is bound by issue, and terms repeated to fill the
+// group cost as much as real ones.  Partial search kernel, k = 3, 512 queries x
+// 24 clusters of 200 docs, us by terms of a query (1 / 2 / 5 / trees of 3-12):
+// row by row 10.4 / 14.1 / 26.2 / 103, groups filled up 20.4 / 18.8 / 29.8 /
+// 50.6, these 11.8 / 14.1 / 22.6 / 46.8.
 template <int K, typename HashesOf>
 __device__ __forceinline__ void eval_term_words(const EvalArgs& a, const Column& c, uint32_t n, HashesOf hashes_of,
                                                 uint64_t (&out)[kTermsAhead<K>]) {
@@ -89,36 +135,15 @@ __device__ __forceinline__ void eval_term_words(const EvalArgs& a, const Column&
 #pragma unroll
     for (int u = 0; u < A; ++u) out[u] = 0;
     if (c.b <= 0 || a.index_numel <= 0) return;
-    uint64_t w[A][K];
-    uint32_t again = 0;  // terms to evaluate position by position
-#pragma unroll
-    for (int u = 0; u < A; ++u) {
-      const ST_EVAL_CONST uint64_t* h = hashes_of(u < n ? u : n - 1);
-      int16_t found[K];
-      bool plain = true;
-#pragma unroll
-      for (int j = 0; j < K; ++j) found[j] = static_cast<int16_t>(fast_mod(h[j], c.fm));
-#pragma unroll
-      for (int j = 0; j < K; ++j) {
-#pragma unroll
-        for (int i = 0; i < j; ++i) plain &= found[i] != found[j];
-        const int64_t at = (c.start + found[j]) * kColumnsPerBundle + c.cib;
-        const bool inside = at >= 0 && at < a.index_numel;
-        plain &= inside;
-        w[u][j] = static_cast<uint64_t>(a.index[inside ? at : 0]);
-      }
-      again |= plain ? 0u : 1u << u;
-    }
-#pragma unroll
-    for (int u = 0; u < A; ++u) {
-      out[u] = w[u][0];
-#pragma unroll
-      for (int j = 1; j < K; ++j) out[u] &= w[u][j];
-    }
-    if (again != 0) {
-#pragma unroll
-      for (int u = 0; u < A; ++u)
-        if ((again >> u) & 1u) out[u] = eval_term_word<K>(a, c, hashes_of(u < n ? u : n - 1));
+    if (n >= A) {
+      eval_term_group<K, A>(a, c, hashes_of, out);
+    } else if (n == 1) {
+      eval_term_group<K, 1>(a, c, hashes_of, out);
+    } else if constexpr (A > 2) {
+      if (n == 2)
+        eval_term_group<K, 2>(a, c, hashes_of, out);
+      else
+        eval_term_group<K, 3>(a, c, hashes_of, out);
     }
   }
 }
@@ -142,17 +167,21 @@ __device__ uint64_t eval_program(const EvalArgs& a, const Column& c,
   };
   constexpr uint32_t A = kTermsAhead<K>;
   uint64_t words[A];
-  if (hdr & kFlatForm) {  // OR of AND-groups: [term ref, negate, group, 0]
-    const ST_EVAL_CONST uint32_t* lit = prog + kProgHeaderWords;
+  if (hdr & kFlatForm) {  // OR of AND-groups: [term ref, negate mask, group mask, 0]
+    typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+    const ST_EVAL_CONST v4* lit = (const ST_EVAL_CONST v4*)(prog + kProgHeaderWords);
     uint64_t res = 0, acc = 0;
-    for (uint32_t j = 0; j < T; j += A, lit += A * kFlatLiteralWords) {
+    for (uint32_t j = 0; j < T; j += A, lit += A) {
       const uint32_t n = T - j < A ? T - j : A;
-      eval_term_words<K>(a, c, n, [&](uint32_t u) { return term_hashes(lit[u * kFlatLiteralWords]); }, words);
+      v4 rec[A];  // whole records at once: one wait for the scalar cache a group
+#pragma unroll
+      for (uint32_t u = 0; u < A; ++u) rec[u] = lit[u < n ? u : n - 1];
+      eval_term_words<K>(a, c, n, [&](uint32_t u) { return term_hashes(rec[u].x); }, words);
 #pragma unroll
       for (uint32_t u = 0; u < A; ++u) {
         if (u >= n) break;
-        const uint64_t neg = lit[u * kFlatLiteralWords + 1] ? ~0ull : 0ull;
-        const uint64_t grp = lit[u * kFlatLiteralWords + 2] ? ~0ull : 0ull;
+        const uint64_t neg = rec[u].y ? ~0ull : 0ull;
+        const uint64_t grp = rec[u].z ? ~0ull : 0ull;
         res |= acc & grp;
         acc = (acc | grp) & (words[u] ^ neg);
       }

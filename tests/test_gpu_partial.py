@@ -114,7 +114,7 @@ def test_partial_random_vs_oracle(seed):
 @pytest.mark.parametrize("bm", [1.1, 40.0])
 def test_partial_terms_read_together(k, hk, bm):
     """Runs and trees of 1-9 terms (rows are read for four terms at a time, for
-    two above k = 5: whole groups and remainders), in bundles so narrow that
+    two above k = 3: whole groups and remainders), in bundles so narrow that
     first positions collide and in wide ones, a first bundle without rows, and
     the same plans on an index cut short (rows outside it read as zero)."""
     rng = np.random.default_rng(100 * k + hk)
