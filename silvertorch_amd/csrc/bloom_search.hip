@@ -78,6 +78,7 @@ constexpr int kBindThreads = 1024;
 constexpr int64_t kDirectReads = 32;
 constexpr int64_t kUnboundWideReads = 240;
 constexpr int64_t kUnboundBoolQueries = 64;
+constexpr uint32_t kUnrolledLiterals = 6;  // of an unbound program (eval_flat: k <= 4)
 constexpr int kBindGrid = 256;     // workgroups of the binding kernel
 // Distinct widths the census tracks.  An index with more gets no slots at
 // all (every bundle resolves its positions itself): whether the table
@@ -506,6 +507,31 @@ bool wide_rows(int64_t bloom_index_numel, int64_t num_bundles) {
   return bloom_index_numel / kColumnsPerBundle > num_bundles * kSearchTileRows;
 }
 
+// Whether unstaged bundles are evaluated faster bound than unbound: at least
+// half of the literals belong to flat programs that the unbound kernel takes a
+// few literals at a time (more than kUnrolledLiterals), in batches whose literal
+// stream is evaluated in rounds (too long for the LDS, where quads would take
+// it), and seven of ten literals have a term of their own (an unbound bundle
+// resolves each term's positions once, which is what binding saves).
+bool long_rounds(const st_search_plan* plan) {
+  if (plan->k_eff < 2 || plan->k_eff > 4) return false;
+  int64_t literals = 0, rounds = 0, terms = 0;
+  for (size_t b = 0; b < plan->batches.size(); ++b) {
+    const SearchBatch& bt = plan->batches[b];
+    if (bt.generic) continue;
+    const std::vector<uint32_t>&insns = plan->batch_insns[b], &starts = plan->batch_starts[b];
+    int64_t in_long = 0;
+    for (const uint32_t s : starts) {
+      const uint32_t hdr = insns[s], n = program_terms(hdr);
+      literals += n;
+      if ((hdr & kFlatForm) && n > kUnrolledLiterals) in_long += n;
+    }
+    terms += bt.num_terms;
+    if (literal_stream_words(*plan, bt, insns, starts) > kQuadStreamMaxWords) rounds += in_long;
+  }
+  return rounds > 0 && 2 * rounds >= literals && 10 * terms >= 7 * literals;
+}
+
 // Validates the arguments and launches the search kernel once per batch.
 void launch_search(const int64_t* bloom_index, int64_t bloom_index_numel,
                    const int64_t* bundle_b_offsets, int64_t num_bundles,
@@ -691,16 +717,27 @@ void compact_zero_offsets(int64_t* row_offsets, int64_t n, hipStream_t s);
 // bundles, 16 queries 31 / 25, 1M docs 64 queries packed 43 / 38, 2M docs 52 /
 // 57; bool output of 256 queries over 1M docs 102 / 152; wide bundles (1,760
 // rows) packed, 4 trees over 12M docs 677 / 531, 16 trees 837 / 1,022, 256
-// trees over 500,000 docs 350 / 305; wide bundles with bool output (never
-// streamed), 64 trees over 2M docs 499 / 324.
+// trees over 500,000 docs 350 / 305.
+// Wide bundles with bool output or counts are never streamed through the LDS;
+// unbound they take 0.3-0.95 of the bound time (64 trees over 2M docs 499 /
+// 324) except where bound rounds keep more rows in flight than the unbound
+// evaluation: long programs (long_rounds) over many bundles, which pay for the
+// binding (16 features of a uniform vocabulary, bool output of 512 queries,
+// bound time over unbound by literals of a query, 8 / 12 / trees of 3-12: k = 3,
+// 6M docs 0.91 / 0.86 / 0.94, 2M docs 0.98 / 0.91 / 0.96, 1.6M docs 1.06 / 1.01 /
+// 1.19; k = 2, 6M docs 0.81 / 0.75 / 0.83; k = 4, 6M docs 0.93 / 0.92 / 0.95, 2M
+// docs 1.01 / 0.98 / 1.01; queries of up to 6 literals 1.2-2.2; trees whose
+// literals repeat terms, k = 4, 8M docs 1.04-1.19).
 extern "C" int st_search_plan_wants_binding(const st_search_plan* plan, int64_t bloom_index_numel,
                                             int64_t num_bundles, int packed_out) {
   using namespace st;
   if (plan == nullptr || num_bundles <= 0) return 0;
   const int64_t cus = device_cu_count();
   const int64_t reads = row_reads(plan);
-  if (wide_rows(bloom_index_numel, num_bundles))
-    return packed_out != 0 && num_bundles > cus && reads > kUnboundWideReads;
+  if (wide_rows(bloom_index_numel, num_bundles)) {
+    if (packed_out != 0) return num_bundles > cus && reads > kUnboundWideReads;
+    return 2 * num_bundles > (plan->k_eff <= 3 ? 7 : 16) * cus && long_rounds(plan);
+  }
   if (reads <= kDirectReads) return 0;
   return num_bundles > 2 * cus || (packed_out == 0 && plan->num_queries > kUnboundBoolQueries);
 }

@@ -1059,6 +1059,30 @@ namespace {
 
 uint64_t align_to(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
+}  // namespace
+
+size_t literal_stream_words(const st_search_plan& plan, const SearchBatch& bt,
+                            const std::vector<uint32_t>& insns, const std::vector<uint32_t>& starts) {
+  const uint32_t* wave_off = reinterpret_cast<const uint32_t*>(plan.blob.data() + bt.off_wave);
+  const int ks = std::max(plan.k_eff, 1);
+  const uint32_t per_block = static_cast<uint32_t>(stream_block_records(ks));
+  size_t total = 0;
+  for (int w = 0; w < kSearchWaves; ++w) {
+    uint32_t n_flat = 0;
+    while (wave_off[w] + n_flat < wave_off[w + 1] && (insns[starts[wave_off[w] + n_flat]] & kFlatForm))
+      ++n_flat;
+    for (uint32_t r0 = 0; r0 < n_flat; r0 += per_block) {
+      const uint32_t n = std::min(per_block, n_flat - r0);
+      uint32_t T = 1;
+      for (uint32_t i = 0; i < n; ++i) T = std::max(T, insns[starts[wave_off[w] + r0 + i]] & 0xFFFFu);
+      total += kRoundHeaderWords + static_cast<size_t>(T) * per_block * bound_record_words(ks);
+    }
+  }
+  return total;
+}
+
+namespace {
+
 // Template of one batch's width block: every bound program (the layout the
 // kernel's per-query loop reads), then the batch's literal stream (absent
 // only when an output row does not fit a record's row field).  Each position word is a code (term,
@@ -1142,18 +1166,7 @@ void build_block_template(const st_search_plan& plan, SearchBatch& bt,
   bt.stream_words = 0;
   bool fits = true;
   // The stream's exact size first, so that it is written in place.
-  size_t stream_total = 0;
-  for (int w = 0; w < kSearchWaves; ++w) {
-    uint32_t n_flat = 0;
-    while (wave_off[w] + n_flat < wave_off[w + 1] && (insns[starts[wave_off[w] + n_flat]] & kFlatForm))
-      ++n_flat;
-    for (uint32_t r0 = 0; r0 < n_flat; r0 += per_block) {
-      const uint32_t n = std::min(per_block, n_flat - r0);
-      uint32_t T = 1;
-      for (uint32_t i = 0; i < n; ++i) T = std::max(T, insns[starts[wave_off[w] + r0 + i]] & 0xFFFFu);
-      stream_total += kRoundHeaderWords + static_cast<size_t>(T) * per_block * srw;
-    }
-  }
+  const size_t stream_total = literal_stream_words(plan, bt, insns, starts);
   size_t at = tmpl.size();
   tmpl.resize(at + stream_total, 0u);
   code.resize(at + stream_total, kTmplCopy);

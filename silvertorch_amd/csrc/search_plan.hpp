@@ -264,3 +264,12 @@ struct st_search_plan {
   // host binding: every bundle has a slot and every slot width is wide
   bool all_wide = false;
 };
+
+namespace st {
+
+// Words of the literal stream of a batch (instructions and program starts as
+// kept for binding), before it is built.
+size_t literal_stream_words(const st_search_plan& plan, const SearchBatch& bt,
+                            const std::vector<uint32_t>& insns, const std::vector<uint32_t>& starts);
+
+}  // namespace st

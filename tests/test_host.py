@@ -300,3 +300,24 @@ def test_partial_response_argument_errors_before_device_work():
         st.bloom_index_search_batch_return_partial_response(idx, bbo, pd, po, co, co, 3, 7, co)
     with pytest.raises(RuntimeError, match="list_bloom_index should not be empty"):
         st.bloom_index_search_batch_return_partial_response_multiple([], [], pd, po, [], [], 3, 7)
+
+
+@pytest.mark.parametrize("k,terms,queries,bundles,packed,want", [
+    # wide bundles (600 rows), bool or counted output: long programs whose
+    # stream does not fit the LDS, over many bundles, are bound; the rest are not
+    (3, 12, 512, 977, False, True), (3, 12, 512, 896, False, False), (3, 12, 512, 782, False, False),
+    (3, 6, 512, 4000, False, False), (3, 12, 64, 4000, False, False), (2, 8, 512, 1465, False, True),
+    (3, 10, 192, 4000, False, False), (3, 10, 200, 4000, False, True),
+    (4, 12, 512, 1465, False, False), (4, 12, 512, 2930, False, True), (5, 12, 512, 4000, False, False),
+    (1, 12, 512, 4000, False, False), (3, 2, 1, 4000, False, False),
+    # packed output of wide bundles: rows named and bundles decide
+    (3, 12, 512, 977, True, True), (3, 12, 512, 256, True, False), (3, 2, 8, 977, True, False),
+])
+def test_binding_rule_of_wide_bundles(k, terms, queries, bundles, packed, want):
+    """st_search_plan_wants_binding at both sides of its limits (on a machine
+    without a GPU the rule assumes 256 CUs)."""
+    texts = [" AND ".join(f"1:{q * terms + t}" for t in range(terms)) for q in range(queries)]
+    _, data, offs = capi.parse_expression_query_batch(texts, 7, True, max(terms, 5))
+    plan = capi.SearchPlan(data, offs, k, 7)
+    got = capi.lib().st_search_plan_wants_binding(plan.handle, bundles * 600 * 32, bundles, int(packed))
+    assert bool(got) is want
