@@ -104,7 +104,8 @@ int st_bloom_build_bundle_offsets(const int64_t* feature_offsets,
  *   feature_offsets   device int64[num_docs * num_features + 1]
  *   feature_values    device int64[num_values]
  *   bundle_b_offsets  device int64[nb + 1] from st_bloom_build_bundle_offsets
- *   max_b             stats[1] of that call (host value)
+ *   max_b             stats[1] of that call (host value): chooses how bundles
+ *                     are split; another value gives the same index
  *   bloom_index       device int64[bloom_index_numel] (output, fully written;
  *                     bloom_index_numel must equal total rows * 32)
  * ------------------------------------------------------------------------- */

@@ -20,6 +20,7 @@
 // (bloom_indexer_cuda.cu:137-251, ~N*b/8 bytes of scratch) are not needed.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "st_common.hpp"
@@ -732,7 +733,10 @@ extern "C" int st_bloom_index_build(const int32_t* feature_ids,
              "null device pointer");
     ST_CHECK(num_values == 0 || feature_values, "feature_values is null");
     set_lds_limits();
-    const ScatterShape shape = scatter_shape(max_b, bloom_index_numel / kColumnsPerBundle, nb);
+    // any max_b gives the same index: one below the widths (a negative one as
+    // zero) sends the wider bundles through global memory
+    const ScatterShape shape =
+        scatter_shape(std::max<int64_t>(max_b, 0), bloom_index_numel / kColumnsPerBundle, nb);
     ScatterArgs a;
     a.feature_ids = feature_ids;
     a.offsets = feature_offsets;

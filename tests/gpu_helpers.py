@@ -19,8 +19,9 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
-def build(ids, offsets, values, b_multiplier: float, k: int):
-    """C-ABI build -> (index, bundle_b_offsets) as numpy arrays."""
+def build(ids, offsets, values, b_multiplier: float, k: int, max_b: int | None = None):
+    """C-ABI build -> (index, bundle_b_offsets) as numpy arrays; max_b in place
+    of the widest bundle's rows."""
     L = capi.lib()
     ids_d = torch.as_tensor(np.ascontiguousarray(ids, dtype=np.int32)).cuda()
     off_d = torch.as_tensor(np.ascontiguousarray(offsets, dtype=np.int64)).cuda()
@@ -37,7 +38,8 @@ def build(ids, offsets, values, b_multiplier: float, k: int):
     index = torch.empty(s[0] * 32, dtype=torch.long, device="cuda")
     capi.check(L.st_bloom_index_build(ids_d.data_ptr(), off_d.data_ptr(),
                                       val_d.data_ptr() if val_d.numel() else None, F, n, val_d.numel(), k,
-                                      bbo.data_ptr(), s[1], index.data_ptr() if index.numel() else None,
+                                      bbo.data_ptr(), s[1] if max_b is None else max_b,
+                                      index.data_ptr() if index.numel() else None,
                                       index.numel(), _stream()))
     torch.cuda.synchronize()
     return index.cpu().numpy(), bbo.cpu().numpy()

@@ -226,6 +226,20 @@ def test_search_op_with_and_without_binding(docs, bm, num_queries):
     np.testing.assert_array_equal(row_offsets.cpu().numpy()[1:], np.cumsum(bits + np.bitwise_count(tail)))
 
 
+@pytest.mark.parametrize("max_b", [-2**62, -1, 0, 1, 100, 2**40])
+def test_build_with_any_max_b(max_b):
+    """max_b of the C entry only chooses the split: negative, too small and too
+    large values give the same index."""
+    rng = np.random.default_rng(11)
+    ids, offs, vals = _random_corpus(rng, 9000, 3, 0, 12, 3000)
+    H.note(f"[build max_b] {max_b}")
+    index, bbo = H.build(ids, offs, vals, 5.0, 3, max_b)
+    want_index, want_bbo = O.bloom_build(ids, offs, vals, 5.0, 3)
+    assert int(np.diff(want_bbo).max()) > 300
+    np.testing.assert_array_equal(bbo, want_bbo)
+    np.testing.assert_array_equal(index, want_index)
+
+
 def test_many_terms_split_into_passes():
     """More distinct terms than one LDS position area holds -> several passes."""
     rng = np.random.default_rng(77)
