@@ -10,17 +10,19 @@
 //   scan_kernel     one workgroup: exclusive prefix sum of the widths into
 //                   bundle_b_offsets, plus the totals the host needs.
 //   scatter_kernel  one workgroup per part of a bundle (16 of its 32 columns,
-//                   fewer for wide bundles or few docs): clears a tile of b
-//                   rows in LDS, hashes every (doc, feature, value) term of
+//                   fewer where bundles are wide or docs few): clears a tile of
+//                   b rows in LDS, hashes every (doc, feature, value) term of
 //                   the part (one thread per value, its place from an LDS map
 //                   of the slot group), ORs its k bits into the tile with LDS
-//                   atomics and stores the tile.  Bundles wider than any tile
-//                   OR straight into global memory.
+//                   atomics and stores the tile.  A bundle too wide for the
+//                   part's tile goes in passes over fewer columns, one that no
+//                   tile holds ORs straight into global memory.
 // The reference's per-doc byte signatures and 64-way transpose
 // (bloom_indexer_cuda.cu:137-251, ~N*b/8 bytes of scratch) are not needed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdint>
 #include <mutex>
 
 #include "st_common.hpp"
@@ -42,7 +44,7 @@ constexpr int kBuildMapBytes = 12288;      // the places of a window's values, i
 constexpr int kBuildMapFeatures = 1 << 20; // features that a 32-bit place names
 constexpr int kBuildQueueWords = 2 * 64;   // a wave's queue of values with colliding positions, in LDS
 constexpr int kBuildStaticLds = 64;        // BundleMod and alignment
-constexpr int kBuildNarrow = 1024;         // mean rows of narrow bundles
+constexpr int kBuildRestLds = 256;         // the same and scatter_rest_kernel's list
 
 // stats layout (int64[6]):
 //   [0] total rows  [1] max bundle width  [2] non-decreasing violation flag
@@ -338,6 +340,21 @@ __device__ __forceinline__ void scatter_value(int64_t k, uint64_t rx, int64_t va
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// LDS of a workgroup besides its tile.
+constexpr int fixed_lds(int threads) {
+  return 8 * kBuildFeatureCache + kBuildMapBytes + 4 * kBuildQueueWords * (threads / 64);
+}
+
+// Words of the tile when a workgroup of `threads` may use `lds` bytes.
+constexpr int tile_words_in(int lds, int threads) { return (lds - fixed_lds(threads)) / 4; }
+
+// The tiles of two workgroups a CU, of one, and of one of scatter_rest_kernel.
+constexpr int kHalfWords = tile_words_in(kLdsBytes / 2 - kBuildStaticLds, kBuildHalfThreads);
+constexpr int kWholeWords = tile_words_in(kLdsBytes - kBuildStaticLds, kBuildThreads);
+constexpr int kRestWords = tile_words_in(kLdsBytes - kBuildRestLds, kBuildThreads);
+
+enum ScatterKind { kScatterEven, kScatterPasses, kScatterRest };
+
 struct ScatterArgs {
   const int32_t* feature_ids;
   const int64_t* offsets;
@@ -349,14 +366,16 @@ struct ScatterArgs {
   int64_t k;
   const int64_t* bundle_b_offsets;
   unsigned long long* index;
-  int lc;         // a workgroup's part of a bundle: 2^lc columns (64 * 2^lc docs)
-  int tile_rows;  // rows its LDS tile holds
+  int lc;          // a workgroup's part of a bundle: 2^lc columns (64 * 2^lc docs)
+  int tile_words;  // 32-bit words of its LDS tile
+  int rest_words;  // one column's words above which a bundle is scatter_rest_kernel's (0: no such launch)
 };
 
 // A tile row: the part's columns as 32-bit words, one word of padding so that
 // the rows' words of one column lie on different LDS banks (64 lanes mostly
 // share a column and differ in the row).
 __host__ __device__ constexpr int tile_stride(int lc) { return (2 << lc) + 1; }
+static_assert(kLdsBytes / (4 * tile_stride(0)) < kBundleModMax, "BundleMod takes every tiled width");
 
 // A value's place, as the slot threads record it in the value map: the doc's
 // bit (doc % 32) in bits 0-4, its 32-bit word in a tile row in bits 5-9 (the
@@ -440,42 +459,31 @@ __device__ __forceinline__ void for_each_value(const ScatterArgs& a, const int64
   }
 }
 
-// One workgroup per part of a bundle (2^lc of its 32 columns).  The tile of
-// the part's rows is cleared in LDS, the part's values are hashed one per
-// thread, their bits ORed into the tile and the tile stored.  The parts of a
-// bundle lie 8 workgroups apart, on one XCD, so that the lines they share
-// meet in its L2.  Parts rather than whole bundles: two tiles fit a CU, so one
-// workgroup hashes while the other clears, loads offsets or stores, and a
-// small corpus (49 bundles at 100,000 docs) still fills the chip.
-// Bound by VALU issue: 242 wave instructions per 64 values at k = 3, one per 4.3
-// cycles (nearly every instruction of the hash, 32-bit multiplies and
-// v_mad_u64_u32 included, takes 4).  100M docs x 4 features, 1.8e9 values, 470
-// rows: 12.0 ms; 17.0 ms with a whole bundle per workgroup (one a CU), the
-// general remainder and 64-bit tile words (315 instructions).  100,000 docs x 2
-// features: 11.8 against 29.9 us.  With 24 waves a CU instead of 16 no faster.
-template <int K>
-__global__ __launch_bounds__(kBuildThreads) void scatter_kernel(ScatterArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
-  __shared__ BundleMod s_mod;
-  const int lc = a.lc, stride = tile_stride(lc);
+// Part `part` of a bundle of b > 0 rows (2^a.lc of its 32 columns): clears the
+// tile of the part's rows in LDS, hashes the part's values one per thread, ORs
+// their bits into the tile and stores it.  Except in an even index, a bundle
+// whose rows the tile does not hold at the part's columns is taken in passes of
+// as many as fit (a pass hashes its own docs only, so that no work is done
+// twice).  The bits of a bundle that the tile does not hold are ORed in global
+// memory, cleared before by this workgroup or (kScatterRest) by scatter_kernel.
+// Ends without a barrier.
+template <int K, ScatterKind kKind>
+__device__ __forceinline__ void scatter_part(const ScatterArgs& a, int64_t bundle, int part, int64_t start,
+                                             int64_t b, uint32_t* lds, BundleMod& s_mod) {
   const int tid = threadIdx.x, T = blockDim.x;
   uint64_t* rxc = reinterpret_cast<uint64_t*>(lds);  // rotl(murmur_mix_x(id), 27)
   uint32_t* vmap = lds + 2 * kBuildFeatureCache;
   uint16_t* vmap16 = reinterpret_cast<uint16_t*>(vmap);
   uint32_t* queues = vmap + kBuildMapBytes / 4;
   uint32_t* tile = queues + kBuildQueueWords * (T >> 6);
-
-  const int parts = 32 >> lc;
-  const int64_t run = blockIdx.x / (8 * parts), at = blockIdx.x % (8 * parts);
-  const int64_t bundle = run * 8 + at % 8;
-  const int part = static_cast<int>(at / 8);
-  if (bundle >= a.num_bundles) return;
-  const int64_t start = a.bundle_b_offsets[bundle];
-  const int64_t b = a.bundle_b_offsets[bundle + 1] - start;
-  if (b <= 0) return;
-  const bool tiled = b <= a.tile_rows;
-  const uint32_t c0 = static_cast<uint32_t>(part) << lc;
-  unsigned long long* gbase = a.index + start * 32 + c0;
+  int lc = a.lc;  // 2^lc columns a pass
+  if constexpr (kKind != kScatterEven) {
+    while (lc > 0 && b * tile_stride(lc) > a.tile_words) --lc;
+  }
+  const bool tiled = b * tile_stride(lc) <= a.tile_words;
+  if (!tiled) lc = a.lc;
+  const int stride = tile_stride(lc);
+  const uint32_t part_begin = static_cast<uint32_t>(part) << a.lc, part_end = part_begin + (1u << a.lc);
   const int64_t F = a.num_features;
   auto rx_id = [&](int64_t f) {
     return rotl64(murmur_mix_x(static_cast<uint64_t>(static_cast<int64_t>(a.feature_ids[f]))), 27);
@@ -485,139 +493,233 @@ __global__ __launch_bounds__(kBuildThreads) void scatter_kernel(ScatterArgs a) {
   if (tiled) {
     for (int i = tid; i < static_cast<int>(lesser(F, kBuildFeatureCache)); i += T) rxc[i] = rx_id(i);
     if (tid == T - 1) s_mod = make_bundle_mod(static_cast<uint32_t>(b));
-    u32x4* clear = reinterpret_cast<u32x4*>(tile);
-    for (int w = tid; w < (static_cast<int>(b) * stride + 3) / 4; w += T) clear[w] = u32x4{0, 0, 0, 0};
-  } else {
-    for (int64_t w = tid; w < words; w += T) gbase[(w >> lc) * 32 + (w & ((1 << lc) - 1))] = 0;
-    __threadfence();
   }
-  __syncthreads();
-
   const int64_t doc0 = bundle * kDocsPerBundle;
   const int64_t docs = lesser(doc0 + kDocsPerBundle, a.num_docs) - doc0;
-  const int64_t dlo = static_cast<int64_t>(c0) * 64;
-  const int64_t dhi = lesser(dlo + (64 << lc), docs);
   const int64_t* offs = a.offsets + doc0 * F;
-  const int64_t slot_lo = dlo * F, slot_hi = dhi > dlo ? dhi * F : slot_lo;
-  if (tiled && F <= kBuildFeatureCache) {
-    TileMod mod{s_mod};
-    mod.m.d = __builtin_amdgcn_readfirstlane(mod.m.d);
-    mod.m.a_lo = __builtin_amdgcn_readfirstlane(mod.m.a_lo);
-    mod.m.a_hi = __builtin_amdgcn_readfirstlane(mod.m.a_hi);
-    mod.m.b_lo = __builtin_amdgcn_readfirstlane(mod.m.b_lo);
-    mod.m.b_hi = __builtin_amdgcn_readfirstlane(mod.m.b_hi);
-    const uint32_t row_bytes = 4 * stride;
-    auto set = [&](uint32_t p, uint32_t m) {
-      atomicOr(reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(tile) +
-                                           (__umul24(p, row_bytes) + 4 * place_word(m))),
-               place_bit(m));
-    };
-    if constexpr (K > 1) {
-      // Values whose first K positions collide (0.6% of the values, but a third
-      // of the waves hold one, at b = 470 and K = 3) wait in the wave's queue
-      // until it is full, and are then hashed again and further together.
-      uint32_t* queue = queues + (tid >> 6) * kBuildQueueWords;
-      const int lane = tid & 63;
-      const int64_t base = slot_hi > slot_lo ? lesser(greater(offs[slot_lo], 0), a.num_values) : 0;
-      int queued = 0;  // wave-uniform
-      auto drain = [&] {
-        if (lane < queued) {
-          const uint32_t i = queue[2 * lane], m = queue[2 * lane + 1];
-          scatter_value<K>(a.k, rxc[place_feature(m)], a.values[base + i], mod, [&](uint32_t p) { set(p, m); });
-        }
-        queued = 0;
-      };
-      for_each_value(a, offs, c0, slot_lo, slot_hi, vmap16, [&](int64_t value, uint32_t m, int64_t index, bool mine) {
-        const uint64_t rx = rxc[place_feature(m)];
-        const uint64_t ry = rotl64(murmur_mix_y(static_cast<uint64_t>(value)), 31);
-        uint32_t found[K];
-        const bool distinct = first_positions<K>(rx, ry, mod, found);
-        if (mine && distinct) {
-#pragma unroll
-          for (int j = 0; j < K; ++j) set(found[j], m);
-        }
-        const bool wait = mine && !distinct;
-        const uint64_t again = __ballot(wait);
-        if (again != 0) {
-          const int more = __popcll(again);
-          if (queued + more > 64) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            drain();
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          }
-          if (wait) {
-            const int at_q = queued + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(again >> 32),
-                                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(again), 0));
-            queue[2 * at_q] = static_cast<uint32_t>(index - base);
-            queue[2 * at_q + 1] = m;
-          }
-          queued += more;
-        }
-      });
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      drain();
-    } else {
-      for_each_value(a, offs, c0, slot_lo, slot_hi, vmap16, [&](int64_t value, uint32_t m, int64_t, bool mine) {
-        if (mine) scatter_value<K>(a.k, rxc[place_feature(m)], value, mod, [&](uint32_t p) { set(p, m); });
-      });
+  for (uint32_t c0 = part_begin; c0 < part_end; c0 += 1u << lc) {
+    unsigned long long* gbase = a.index + start * 32 + c0;
+    if (tiled) {
+      if (c0 != part_begin) __syncthreads();  // the last pass's tile is stored
+      u32x4* clear = reinterpret_cast<u32x4*>(tile);
+      for (int w = tid; w < (static_cast<int>(b) * stride + 3) / 4; w += T) clear[w] = u32x4{0, 0, 0, 0};
+    } else if constexpr (kKind != kScatterRest) {
+      for (int64_t w = tid; w < words; w += T) gbase[(w >> lc) * 32 + (w & ((1 << lc) - 1))] = 0;
+      __threadfence();
     }
-  } else {
-    // A bundle wider than the tile (its bits go straight to global memory),
-    // or more features than the cache or than a place names (a thread per
-    // slot then).
-    const WideMod mod{make_fastmod(static_cast<uint64_t>(b))};
-    auto one = [&](int64_t value, int64_t f, uint32_t word, uint32_t doc) {
-      scatter_value<K>(a.k, rx_id(f), value, mod, [&](uint32_t p) {
-        if (tiled) {
-          atomicOr(tile + (p * stride + word), 0x80000000u >> doc);
-        } else {
-          atomicOr(gbase + static_cast<uint64_t>(p) * 32 + (word >> 1),
-                   1ull << (((word & 1u) << 5) + 31u - doc));
-        }
-      });
-    };
-    if (F < kBuildMapFeatures) {
-      for_each_value(a, offs, c0, slot_lo, slot_hi, vmap, [&](int64_t value, uint32_t m, int64_t, bool mine) {
-        if (mine) one(value, place_feature(m), place_word(m), m & 31u);
-      });
+    __syncthreads();
+    const int64_t dlo = static_cast<int64_t>(c0) * 64;
+    const int64_t dhi = lesser(dlo + (64 << lc), docs);
+    const int64_t slot_lo = dlo * F, slot_hi = dhi > dlo ? dhi * F : slot_lo;
+    if (tiled && F <= kBuildFeatureCache) {
+      TileMod mod{s_mod};
+      mod.m.d = __builtin_amdgcn_readfirstlane(mod.m.d);
+      mod.m.a_lo = __builtin_amdgcn_readfirstlane(mod.m.a_lo);
+      mod.m.a_hi = __builtin_amdgcn_readfirstlane(mod.m.a_hi);
+      mod.m.b_lo = __builtin_amdgcn_readfirstlane(mod.m.b_lo);
+      mod.m.b_hi = __builtin_amdgcn_readfirstlane(mod.m.b_hi);
+      const uint32_t row_bytes = 4 * stride;
+      auto set = [&](uint32_t p, uint32_t m) {
+        atomicOr(reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(tile) +
+                                             (__umul24(p, row_bytes) + 4 * place_word(m))),
+                 place_bit(m));
+      };
+      if constexpr (K > 1) {
+        // Values whose first K positions collide (0.6% of the values, but a third
+        // of the waves hold one, at b = 470 and K = 3) wait in the wave's queue
+        // until it is full, and are then hashed again and further together.
+        uint32_t* queue = queues + (tid >> 6) * kBuildQueueWords;
+        const int lane = tid & 63;
+        const int64_t base = slot_hi > slot_lo ? lesser(greater(offs[slot_lo], 0), a.num_values) : 0;
+        int queued = 0;  // wave-uniform
+        auto drain = [&] {
+          if (lane < queued) {
+            const uint32_t i = queue[2 * lane], m = queue[2 * lane + 1];
+            scatter_value<K>(a.k, rxc[place_feature(m)], a.values[base + i], mod, [&](uint32_t p) { set(p, m); });
+          }
+          queued = 0;
+        };
+        for_each_value(a, offs, c0, slot_lo, slot_hi, vmap16, [&](int64_t value, uint32_t m, int64_t index, bool mine) {
+          const uint64_t rx = rxc[place_feature(m)];
+          const uint64_t ry = rotl64(murmur_mix_y(static_cast<uint64_t>(value)), 31);
+          uint32_t found[K];
+          const bool distinct = first_positions<K>(rx, ry, mod, found);
+          if (mine && distinct) {
+#pragma unroll
+            for (int j = 0; j < K; ++j) set(found[j], m);
+          }
+          const bool wait = mine && !distinct;
+          const uint64_t again = __ballot(wait);
+          if (again != 0) {
+            const int more = __popcll(again);
+            if (queued + more > 64) {
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+              drain();
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+            if (wait) {
+              const int at_q = queued + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(again >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(again), 0));
+              queue[2 * at_q] = static_cast<uint32_t>(index - base);
+              queue[2 * at_q + 1] = m;
+            }
+            queued += more;
+          }
+        });
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        drain();
+      } else {
+        for_each_value(a, offs, c0, slot_lo, slot_hi, vmap16, [&](int64_t value, uint32_t m, int64_t, bool mine) {
+          if (mine) scatter_value<K>(a.k, rxc[place_feature(m)], value, mod, [&](uint32_t p) { set(p, m); });
+        });
+      }
     } else {
-      for (int64_t rel = slot_lo + tid; rel < slot_hi; rel += T) {
-        const int64_t d = rel / F, f = rel - d * F;
-        const int64_t v0 = lesser(greater(offs[rel], 0), a.num_values);
-        const int64_t v1 = lesser(greater(offs[rel + 1], 0), a.num_values);
-        for (int64_t v = v0; v < v1; ++v)
-          one(a.values[v], f, static_cast<uint32_t>(((d >> 5) ^ 1) - 2 * c0), static_cast<uint32_t>(d & 31));
+      // A bundle wider than the tile (its bits go straight to global memory),
+      // or more features than the cache (300,000 docs of 60 features and 3 or 12
+      // values 0.140 and 0.160 ms, of 65 features 0.150 and 0.175 ms) or than a
+      // place names (a thread per slot then).
+      uint64_t width = static_cast<uint64_t>(b);
+      asm volatile("" : "+s"(width));  // formed here: hoisted, its registers would spill the other path's
+      const WideMod mod{make_fastmod(width)};
+      auto one = [&](int64_t value, int64_t f, uint32_t word, uint32_t doc) {
+        scatter_value<K>(a.k, rx_id(f), value, mod, [&](uint32_t p) {
+          if (tiled) {
+            atomicOr(tile + (p * stride + word), 0x80000000u >> doc);
+          } else {
+            atomicOr(gbase + static_cast<uint64_t>(p) * 32 + (word >> 1),
+                     1ull << (((word & 1u) << 5) + 31u - doc));
+          }
+        });
+      };
+      if (F < kBuildMapFeatures) {
+        for_each_value(a, offs, c0, slot_lo, slot_hi, vmap, [&](int64_t value, uint32_t m, int64_t, bool mine) {
+          if (mine) one(value, place_feature(m), place_word(m), m & 31u);
+        });
+      } else {
+        for (int64_t rel = slot_lo + tid; rel < slot_hi; rel += T) {
+          const int64_t d = rel / F, f = rel - d * F;
+          const int64_t v0 = lesser(greater(offs[rel], 0), a.num_values);
+          const int64_t v1 = lesser(greater(offs[rel + 1], 0), a.num_values);
+          for (int64_t v = v0; v < v1; ++v)
+            one(a.values[v], f, static_cast<uint32_t>(((d >> 5) ^ 1) - 2 * c0), static_cast<uint32_t>(d & 31));
+        }
       }
     }
+    if (!tiled) return;
+    __syncthreads();
+    for (int w = tid; w < static_cast<int>(words); w += T) {
+      const int p = w >> lc, c = w & ((1 << lc) - 1);
+      const uint32_t* src = tile + p * stride + 2 * c;
+      const unsigned long long v = (static_cast<unsigned long long>(src[1]) << 32) | src[0];
+      unsigned long long* dst = gbase + static_cast<int64_t>(p) * 32 + c;
+      // whole 128-byte lines stream past the caches; parts of a line meet in L2
+      if (lc >= 4) __builtin_nontemporal_store(v, dst);
+      else *dst = v;
+    }
+    if constexpr (kKind == kScatterEven) return;
   }
-  if (!tiled) return;
-  __syncthreads();
-  for (int w = tid; w < static_cast<int>(words); w += T) {
-    const int p = w >> lc, c = w & ((1 << lc) - 1);
-    const uint32_t* src = tile + p * stride + 2 * c;
-    const unsigned long long v = (static_cast<unsigned long long>(src[1]) << 32) | src[0];
-    unsigned long long* dst = gbase + static_cast<int64_t>(p) * 32 + c;
-    // whole 128-byte lines stream past the caches; parts of a line meet in L2
-    if (lc >= 4) __builtin_nontemporal_store(v, dst);
-    else *dst = v;
+}
+
+// One workgroup per part of a bundle (2^lc of its 32 columns).  The parts of a
+// bundle lie 8 workgroups apart, on one XCD, so that the lines they share
+// meet in its L2.  Parts rather than whole bundles: two tiles fit a CU, so one
+// workgroup hashes while the other clears, loads offsets or stores, and a
+// small corpus (49 bundles at 100,000 docs) still fills the chip.
+// kScatterPasses: some bundles are wider than the tile holds at the part's
+// columns; the loop over passes costs the others 2-8% (registers), so that
+// indices without such bundles run without it.  What scatter_rest_kernel ORs in
+// global memory is cleared here, whole rows by each workgroup.
+// Bound by VALU issue: 242 wave instructions per 64 values at k = 3, one per 4.3
+// cycles (nearly every instruction of the hash, 32-bit multiplies and
+// v_mad_u64_u32 included, takes 4).  100M docs x 4 features, 1.8e9 values, 470
+// rows: 12.0 ms; 17.0 ms with a whole bundle per workgroup (one a CU), the
+// general remainder and 64-bit tile words (315 instructions).  100,000 docs x 2
+// features: 11.8 against 29.9 us.
+template <int K, ScatterKind kKind>
+__global__ __launch_bounds__(kBuildThreads) void scatter_kernel(ScatterArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  __shared__ BundleMod s_mod;
+  const int parts = 32 >> a.lc;
+  const int64_t run = blockIdx.x / (8 * parts), at = blockIdx.x % (8 * parts);
+  const int64_t bundle = run * 8 + at % 8;
+  const int part = static_cast<int>(at / 8);
+  if (bundle >= a.num_bundles) return;
+  const int64_t start = a.bundle_b_offsets[bundle];
+  const int64_t b = a.bundle_b_offsets[bundle + 1] - start;
+  if (b <= 0) return;
+  if constexpr (kKind == kScatterPasses) {
+    if (a.rest_words != 0 && b * tile_stride(0) > a.rest_words) {
+      if (b * tile_stride(0) > kRestWords) {
+        const int64_t end = (start + b * (part + 1) / parts) * 32;
+        for (int64_t w = (start + b * part / parts) * 32 + threadIdx.x; w < end; w += blockDim.x)
+          __builtin_nontemporal_store(0ull, a.index + w);
+      }
+      return;
+    }
+  }
+  scatter_part<K, kKind>(a, bundle, part, start, b, lds, s_mod);
+}
+
+// The bundles that scatter_kernel's tile does not hold at any number of columns,
+// with the tile of a whole CU: persistent workgroups, each of which looks all
+// bundle widths through (1,024 at a time) and takes its share of the wide
+// bundles' parts.  The parts of a bundle are taken on one XCD (workgroup i runs
+// on XCD i % 8; the n-th wide bundle is XCD n % 8's).
+template <int K>
+__global__ __launch_bounds__(kBuildThreads) void scatter_rest_kernel(ScatterArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+  __shared__ BundleMod s_mod;
+  __shared__ unsigned long long wide[kBuildThreads / 64];  // bundles of the 1,024, by wave and lane
+  const int tid = threadIdx.x;
+  const int64_t parts = 32 >> a.lc, xcd = blockIdx.x % 8, per_xcd = gridDim.x / 8;
+  // this workgroup's next part of its XCD's wide bundles; wide bundles before the 1,024
+  int64_t item = blockIdx.x / 8, seen = 0;
+  for (int64_t base = 0; base < a.num_bundles; base += kBuildThreads) {
+    const int64_t i = base + tid;
+    const int64_t b = i < a.num_bundles ? a.bundle_b_offsets[i + 1] - a.bundle_b_offsets[i] : 0;
+    const uint64_t mask = __ballot(b * tile_stride(0) > a.rest_words);
+    __syncthreads();  // the last 1,024's readers are done
+    if ((tid & 63) == 0) wide[tid >> 6] = mask;
+    __syncthreads();
+    int64_t n = 0;
+    for (int w = 0; w < kBuildThreads / 64; ++w) n += __popcll(wide[w]);
+    for (; item / parts * 8 + xcd < seen + n; item += per_xcd) {
+      int nth = static_cast<int>(item / parts * 8 + xcd - seen), w = 0;
+      while (nth >= __popcll(wide[w])) nth -= __popcll(wide[w++]);
+      uint64_t m = wide[w];
+      for (; nth > 0; --nth) m &= m - 1;
+      const int64_t bundle = base + 64 * w + __builtin_ctzll(m);
+      const int64_t start = a.bundle_b_offsets[bundle];
+      scatter_part<K, kScatterRest>(a, bundle, static_cast<int>(item % parts), start,
+                                    a.bundle_b_offsets[bundle + 1] - start, lds, s_mod);
+      __syncthreads();  // the tile is stored
+    }
+    seen += n;
   }
 }
 
 using ScatterFn = void (*)(ScatterArgs);
 
-ScatterFn select_scatter(int64_t k) {
+template <int K>
+ScatterFn scatter_of(ScatterKind kind) {
+  return kind == kScatterRest ? scatter_rest_kernel<K>
+         : kind == kScatterPasses ? scatter_kernel<K, kScatterPasses>
+                                  : scatter_kernel<K, kScatterEven>;
+}
+
+ScatterFn select_scatter(int64_t k, ScatterKind kind) {
   switch (k) {
-    case 1: return scatter_kernel<1>;
-    case 2: return scatter_kernel<2>;
-    case 3: return scatter_kernel<3>;
-    case 4: return scatter_kernel<4>;
-    case 5: return scatter_kernel<5>;
-    case 6: return scatter_kernel<6>;
-    case 7: return scatter_kernel<7>;
-    case 8: return scatter_kernel<8>;
-    case 9: return scatter_kernel<9>;
-    case 10: return scatter_kernel<10>;
-    default: return scatter_kernel<0>;
+    case 1: return scatter_of<1>(kind);
+    case 2: return scatter_of<2>(kind);
+    case 3: return scatter_of<3>(kind);
+    case 4: return scatter_of<4>(kind);
+    case 5: return scatter_of<5>(kind);
+    case 6: return scatter_of<6>(kind);
+    case 7: return scatter_of<7>(kind);
+    case 8: return scatter_of<8>(kind);
+    case 9: return scatter_of<9>(kind);
+    case 10: return scatter_of<10>(kind);
+    default: return scatter_of<0>(kind);
   }
 }
 
@@ -633,10 +735,12 @@ void set_lds_limits() {
   static hipError_t status = hipSuccess;
   std::call_once(once, [] {
     for (int64_t k = 0; k <= 10; ++k) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(select_scatter(k)),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               kLdsBytes - kBuildStaticLds);
-      if (e != hipSuccess && status == hipSuccess) status = e;
+      for (const ScatterKind kind : {kScatterEven, kScatterPasses, kScatterRest}) {
+        const hipError_t e = hipFuncSetAttribute(
+            reinterpret_cast<const void*>(select_scatter(k, kind)), hipFuncAttributeMaxDynamicSharedMemorySize,
+            kLdsBytes - (kind == kScatterRest ? kBuildRestLds : kBuildStaticLds));
+        if (e != hipSuccess && status == hipSuccess) status = e;
+      }
     }
   });
   if (status != hipSuccess)
@@ -644,38 +748,43 @@ void set_lds_limits() {
 }
 
 struct ScatterShape {
-  int lc, tile_rows, threads, lds;
+  int lc, tile_words, threads;
+  bool passes;  // some bundle is wider than the tile holds at 2^lc columns
+  bool rest;    // ... than it holds at one column
 };
 
-// LDS of a workgroup besides its tile.
-int fixed_lds(int threads) {
-  return 8 * kBuildFeatureCache + kBuildMapBytes + 4 * kBuildQueueWords * (threads / 64);
-}
-
-// Rows a tile holds when a workgroup of `threads` may use `lds` bytes.
-int tile_rows_in(int lds, int threads, int lc) {
-  return (lds - kBuildStaticLds - fixed_lds(threads)) / (4 * tile_stride(lc));
-}
-
-// The part of a bundle a workgroup takes: as many columns as let two tiles of
-// the widest bundle share a CU (16 columns up to 492 rows, 8 up to 955, 4 up
-// to 1,804), else as many as fit the whole CU (4 up to 3,966 rows, 2 up to
-// 7,139, 1 up to 11,898).  Where a few bundles are that wide among narrow ones
-// (mean below kBuildNarrow), the parts keep 8 columns and the bundles that no
-// tile holds OR into global memory, as bundles wider than any tile do (1M docs
-// of up to 96 values, k = 5, 3,900-4,300 rows: 11.0 ms so, 0.94 ms in 2-column
-// tiles).  A corpus too small to give every CU two workgroups is split further.
+// The part of a bundle a workgroup takes: as many columns as let two tiles of a
+// typical bundle share a CU (16 columns up to 492 rows, 8 up to 955, 4 up to
+// 1,804), else as many as fit the whole CU (4 up to 3,966 rows, 2 up to 7,139, 1
+// up to 11,898).  Typical is a quarter above the mean width, or the widest where
+// that is less: a few wide bundles among narrow ones go in passes, and those
+// that the tile does not hold at one column (5,413 or 11,898 rows) in a launch
+// of their own, so that they do not change the parts of the others.
+// 20M docs of 1-2 values (20 rows), 2% of the bundles wider, ms by their rows
+// (1,200 / 3,000 / 6,000 / 12,500): parts for the widest bundle 1.15 / 2.14 /
+// 1.68 / 1.80, these 0.60 / 0.74 / 0.79 / 0.95, without wide bundles 0.49.
+// 1M docs of 8 features, a fifth of the bundles 3,000 rows: 0.284 -> 0.241; all
+// bundles 12,500 rows: 3.67 -> 2.77 (whole rows cleared, 16 parts OR).
+// A corpus too small to give every CU two workgroups is split further.
 ScatterShape scatter_shape(int64_t max_b, int64_t total_rows, int64_t nb) {
-  ScatterShape s{3, tile_rows_in(kLdsBytes, kBuildThreads, 3), kBuildThreads, 0};
-  const bool wide = total_rows >= kBuildNarrow * nb;
-  for (int lc = wide ? 0 : 2; lc <= 2; ++lc)
-    if (max_b <= tile_rows_in(kLdsBytes, kBuildThreads, lc)) s = {lc, static_cast<int>(max_b), kBuildThreads, 0};
+  const int64_t widest = std::min<int64_t>(max_b, INT32_MAX);
+  const int64_t typical = std::min(widest, (total_rows + nb - 1) / nb * 5 / 4);
+  ScatterShape s{0, kWholeWords, kBuildThreads, false, false};
+  for (int lc = 1; lc <= 2; ++lc)
+    if (typical * tile_stride(lc) <= kWholeWords) s.lc = lc;
   for (int lc = 2; lc <= 4; ++lc)
-    if (max_b <= tile_rows_in(kLdsBytes / 2, kBuildHalfThreads, lc))
-      s = {lc, static_cast<int>(max_b), kBuildHalfThreads, 0};
+    if (typical * tile_stride(lc) <= kHalfWords) s = {lc, kHalfWords, kBuildHalfThreads, false, false};
   while (s.lc > 2 && s.threads == kBuildHalfThreads && nb * (32 >> s.lc) < 2 * cu_count()) --s.lc;
-  s.lds = fixed_lds(s.threads) + (4 * tile_stride(s.lc) * s.tile_rows + 15) / 16 * 16;
+  s.passes = widest * tile_stride(s.lc) > s.tile_words;
+  s.rest = widest * tile_stride(0) > s.tile_words;
+  if (!s.passes) s.tile_words = static_cast<int>(widest) * tile_stride(s.lc);
   return s;
+}
+
+void launch_scatter(ScatterArgs a, ScatterKind kind, int64_t grid, int threads, hipStream_t s) {
+  const int lds = fixed_lds(threads) + (4 * a.tile_words + 15) / 16 * 16;
+  hipLaunchKernelGGL(select_scatter(a.k, kind), dim3(static_cast<unsigned>(grid)), dim3(threads), lds, s, a);
+  check_launch(kind == kScatterRest ? "scatter_rest_kernel" : "scatter_kernel");
 }
 
 }  // namespace
@@ -749,11 +858,15 @@ extern "C" int st_bloom_index_build(const int32_t* feature_ids,
     a.index = reinterpret_cast<unsigned long long*>(bloom_index);
     a.num_bundles = nb;
     a.lc = shape.lc;
-    a.tile_rows = shape.tile_rows;
+    a.tile_words = shape.tile_words;
+    a.rest_words = shape.rest ? shape.tile_words : 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t grid = (nb + 7) / 8 * 8 * (32 >> shape.lc);
-    hipLaunchKernelGGL(select_scatter(k), dim3(static_cast<unsigned>(grid)), dim3(shape.threads),
-                       shape.lds, s, a);
-    check_launch("scatter_kernel");
+    launch_scatter(a, shape.passes ? kScatterPasses : kScatterEven, (nb + 7) / 8 * 8 * (32 >> shape.lc),
+                   shape.threads, s);
+    if (shape.rest) {
+      a.lc = 1;
+      a.tile_words = kRestWords;
+      launch_scatter(a, kScatterRest, std::max(8, cu_count() / 8 * 8), kBuildThreads, s);
+    }
   });
 }

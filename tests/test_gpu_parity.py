@@ -169,61 +169,64 @@ def test_build_feature_counts_vs_oracle(F, n):
                                        torch.from_numpy(vals).cuda(), 2.0, 3)
 
 
-# Widest bundle's rows on both sides of each tile limit (492, 955 and 1,804
-# rows with half a CU, 3,966, 7,139 and 11,898 with a whole one, then global
-# memory; beyond 3,966 narrow tiles only where the mean width is large: docs
-# in one or two bundles).
-@pytest.mark.parametrize("widest", [2, 492, 494, 954, 956, 1804, 1806, 3966, 3968, 7138, 7140, 11898, 11904])
-@pytest.mark.parametrize("docs,F", [(4097, 3), (4097, 64), (1500, 2), (4097, 65), (530_001, 1)])
-def test_build_tile_shapes_vs_oracle(widest, docs, F):
-    """Every split of a bundle over workgroups (by the widest bundle and by
-    the number of bundles), value counts from none to many per slot, one bundle
-    wider than the rest."""
-    k, bm = (1, 2.0) if widest % 4 else (2, 1.001)
+# Widest bundle's rows on both sides of each tile limit: 492, 955, 1,804, 3,248
+# and 5,413 rows at 16 to 1 columns with two tiles a CU, 3,966, 7,139 and 11,898
+# at 4 to 1 columns with one, 11,882 where such bundles have a launch of their
+# own; then global memory.
+@pytest.mark.parametrize("widest", [2, 3, 492, 493, 955, 956, 1804, 1805, 3248, 3249, 3966, 3967, 5413, 5414, 7139,
+                                    7140, 11882, 11883, 11898, 11899])
+@pytest.mark.parametrize("docs,F,wide", [(4097, 3, "one"), (4097, 64, "one"), (1500, 2, "one"), (4097, 65, "one"),
+                                         (530_001, 1, "one"), (4097, 2, "all"), (40_000, 1, "some"),
+                                         (530_001, 1, "all")])
+def test_build_tile_shapes_vs_oracle(widest, docs, F, wide):
+    """Every split of a bundle over workgroups (by the mean width, the widest
+    and the number of bundles), value counts from none to many per slot: one
+    bundle of exactly `widest` rows among narrow ones, every third one, or all."""
+    if wide == "all" and widest > 2000:
+        docs = min(docs, 12_000)  # not an index of gigabytes
+    k = 1 + widest % 2
+    most = max(1, widest // (2 * k))
+    bm = (widest + 0.5) / (most * k)
     rng = np.random.default_rng(widest + docs + F)
-    counts = (rng.random(docs * F) < (1.5 / F)).astype(np.int64)
-    most = -(-widest // 2)
-    doc = int(rng.integers(0, docs))  # the doc that makes its bundle the widest
-    counts.reshape(docs, F)[doc] = 0
-    at = np.sort(rng.integers(0, F, most))
-    np.add.at(counts.reshape(docs, F)[doc], at, 1)
-    offs = np.concatenate([[0], np.cumsum(counts)])
+    counts = np.zeros((docs, F), dtype=np.int64)
+    if wide != "all":
+        counts[rng.random((docs, F)) < 1.5 / F] = 1
+        counts[counts.sum(1) > most] = 0
+    nb = -(-docs // 2048)
+    for bundle in {"one": [int(rng.integers(0, nb))], "some": range(0, nb, 3), "all": range(nb)}[wide]:
+        doc = min(docs - 1, bundle * 2048 + int(rng.integers(0, 2048)))
+        counts[doc] = 0
+        np.add.at(counts[doc], rng.integers(0, F, most), 1)
+    offs = np.concatenate([[0], np.cumsum(counts.reshape(-1))])
     vals = rng.integers(-2**62, 2**62, int(offs[-1]))
     ids = np.arange(1, F + 1, dtype=np.int32) * 7
-    H.note(f"[build tiles] widest={widest} docs={docs} F={F} k={k}")
+    H.note(f"[build tiles] widest={widest} docs={docs} F={F} k={k} wide={wide}")
     index, bbo = H.build(ids, offs, vals, bm, k)
     want_index, want_bbo = O.bloom_build(ids, offs, vals, bm, k)
     np.testing.assert_array_equal(bbo, want_bbo)
     np.testing.assert_array_equal(index, want_index)
-    assert int(np.diff(bbo).max()) >= widest
+    assert int(np.diff(bbo).max()) == widest
 
 
-@pytest.mark.parametrize("docs,bm", [(9000, 5.0), (9000, 60.0), (9000, 200.0), (1_050_000, 5.0), (530_000, 60.0)])
-@pytest.mark.parametrize("num_queries", [1, 9, 64, 65, 130])
-def test_search_op_with_and_without_binding(docs, bm, num_queries):
-    """The operator's choice of a bound or an unbound plan (and of rows read
-    without a tile for a term or two) at both sides of its limits: 9,000 docs
-    are 5 bundles, 1,050,000 are 513; b is ~50, ~600 (wider than the tile) or
-    ~2,000 rows; packed, bool and counted outputs against the oracle."""
-    rng = np.random.default_rng(docs + num_queries)
-    ids, offs, vals = _random_corpus(rng, docs, 2, 0, 3, 40)
-    index, bbo = O.bloom_build(ids, offs, vals, bm, 2)
-    term = lambda: ("NOT " if rng.random() < 0.2 else "") + f"{int(rng.choice(ids))}:{int(rng.integers(0, 45))}"
-    queries = [term() if i % 3 == 0 else f"{term()} AND ({term()} OR {term()})" for i in range(num_queries)]
-    pd, po = _plans(queries, 5, 5)
-    want = O.search_packed(index, bbo, pd, po, 2, 5)
-    H.note(f"[op binding] docs={docs} bm={bm} queries={num_queries}")
-    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (index, bbo)]
-    plans = [torch.from_numpy(np.ascontiguousarray(a)) for a in (pd, po)]
-    got = torch.ops.st.bloom_index_search_batch(*t, *plans, 2, 5, False).cpu().numpy()
-    np.testing.assert_array_equal(got, want)
-    if docs * num_queries < 40_000_000:
-        mask = torch.ops.st.bloom_index_search_batch(*t, *plans, 2, 5, True).cpu().numpy()
-        np.testing.assert_array_equal(mask, O.unpack_bool(want))
-    _, row_offsets = torch.ops.st.bloom_index_search_batch_ids(*t, *plans, 2, 5, docs)
-    bits = np.bitwise_count(want.view(np.uint64)[:, :docs // 64]).sum(1, dtype=np.int64)
-    tail = want.view(np.uint64)[:, docs // 64] >> np.uint64(64 - docs % 64) if docs % 64 else np.zeros(1, np.uint64)
-    np.testing.assert_array_equal(row_offsets.cpu().numpy()[1:], np.cumsum(bits + np.bitwise_count(tail)))
+@pytest.mark.parametrize("docs,k,values", [(4500, 10, 5), (4500, 10, 60), (4500, 7, 40), (530_000, 3, 3), (530_000, 5, 2)])
+def test_build_collision_queue_vs_oracle(docs, k, values):
+    """Bundles so narrow for k that many terms' first positions collide: each
+    wave's queue of 64 such values fills and is emptied within a pass."""
+    rng = np.random.default_rng(k)
+    bm = 1.01
+    offs = np.arange(docs + 1, dtype=np.int64) * values
+    vals = rng.integers(-2**62, 2**62, docs * values)
+    ids = np.array([5], dtype=np.int32)
+    b = int(float(values * k) * bm)
+    distinct = float(np.prod(1 - np.arange(k) / b))
+    columns = 4 if docs < 500_000 else 16  # of a part, taken by 8 waves
+    waiting = (1 - distinct) * columns * 64 * values / 8
+    H.note(f"[build queue] k={k} b={b}: {waiting:.0f} values wait in a wave")
+    assert waiting > 90
+    index, bbo = H.build(ids, offs, vals, bm, k)
+    want_index, want_bbo = O.bloom_build(ids, offs, vals, bm, k)
+    np.testing.assert_array_equal(bbo, want_bbo)
+    np.testing.assert_array_equal(index, want_index)
 
 
 @pytest.mark.parametrize("max_b", [-2**62, -1, 0, 1, 100, 2**40])
