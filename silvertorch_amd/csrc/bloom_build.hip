@@ -765,7 +765,9 @@ struct ScatterShape {
 // 1.68 / 1.80, these 0.60 / 0.74 / 0.79 / 0.95, without wide bundles 0.49.
 // 1M docs of 8 features, a fifth of the bundles 3,000 rows: 0.284 -> 0.241; all
 // bundles 12,500 rows: 3.67 -> 2.77 (whole rows cleared, 16 parts OR).
-// A corpus too small to give every CU two workgroups is split further.
+// A corpus too small to give every CU two workgroups is split further, one of
+// over half a million bundles less far than its widths ask for where the grid
+// would pass 2^32 threads (the passes do the rest).
 ScatterShape scatter_shape(int64_t max_b, int64_t total_rows, int64_t nb) {
   const int64_t widest = std::min<int64_t>(max_b, INT32_MAX);
   const int64_t typical = std::min(widest, (total_rows + nb - 1) / nb * 5 / 4);
@@ -775,6 +777,7 @@ ScatterShape scatter_shape(int64_t max_b, int64_t total_rows, int64_t nb) {
   for (int lc = 2; lc <= 4; ++lc)
     if (typical * tile_stride(lc) <= kHalfWords) s = {lc, kHalfWords, kBuildHalfThreads, false, false};
   while (s.lc > 2 && s.threads == kBuildHalfThreads && nb * (32 >> s.lc) < 2 * cu_count()) --s.lc;
+  while (s.lc < 4 && (nb + 7) / 8 * 8 * (32 >> s.lc) * s.threads > int64_t{UINT32_MAX}) ++s.lc;
   s.passes = widest * tile_stride(s.lc) > s.tile_words;
   s.rest = widest * tile_stride(0) > s.tile_words;
   if (!s.passes) s.tile_words = static_cast<int>(widest) * tile_stride(s.lc);
