@@ -757,29 +757,47 @@ void set_lds_limits() {
     throw Error(ST_ERR_HIP, cat("hipFuncSetAttribute failed: ", hipGetErrorString(status)));
 }
 
-// Doc ranges of the rounds (aligned to bundles): a first round without a
-// threshold, then each round `growth` times everything before it, which leaves
-// about growth x topk candidates per query.  A round takes about 20 us of fixed
-// time and a candidate about 0.4 ns, so growth lies where a round's candidates
-// cost a few rounds (kRoundCandidates over all queries), between 8 (512 queries
-// of 100: 2.9-3.0 ms; x4 and x12 no faster) and half of what the selection
-// holds in LDS (16 queries of 10 over 200,000 docs: two rounds instead of
-// three).  512 queries of 10 over 1M docs: 0.29 ms with x8, 0.72 ms with x204.
-// In the safe schedule no round is larger than the candidate segments can
-// always hold.
-std::vector<int64_t> round_bounds(int64_t num_docs, int64_t num_queries, int64_t topk, bool safe) {
-  std::vector<int64_t> b{0};
-  int64_t pos = 0;
+// A call's rounds: one of `first` docs without a threshold, then each `growth`
+// times everything before it.
+struct Schedule {
+  int64_t first;
+  double growth;
+};
+
+// A round after the first leaves about growth x topk
+// candidates per query where docs lie in random order.  A round takes about
+// 20 us of fixed time; a candidate costs its tile's slow path, and more where the
+// staged kernel's waves hold more queries.  Over 1-512 queries of 200,000-8M
+// docs, each time over the better of the two schedules that this one took the
+// place of (8,192 docs and x8; 2,048 and up to x2,048): read directly, top 1 and
+// 10 x128 0.89-1.02 (x512 up to 1.95), top 50 x32 0.97-1.04; staged, top 1 x32
+// 0.97-1.04 (x512 1.0-1.6), top 10 x16 1.03-1.08 (x128 1.04-1.2), top 50 and 100
+// 8,192 and x8 1.00-1.06 (2,048 and x16 1.08-1.15).
+// Read directly, the rounds that a growth gives grow by equal factors, which
+// leaves the fewest candidates; staged this measured 0-4% slower.
+Schedule first_schedule(bool few, int64_t num_queries, int64_t num_docs, int64_t topk) {
+  const int64_t first = topk <= (few || num_docs < int64_t{1} << 20 ? 64 : 16) ? 2048 : 8192;
+  if (!few && num_docs >= int64_t{1} << 20) return {first, topk <= 4 ? 32.0 : topk <= 16 ? 16.0 : 8.0};
+  int64_t growth = std::min(kSelectSlots / 2 / topk, kRoundCandidates / (num_queries * topk));
+  growth = std::max<int64_t>(8, std::min(growth, std::max<int64_t>(256, 2048 / num_queries)));
+  if (!few) return {first, static_cast<double>(growth)};
+  const double all = std::max(1.0, static_cast<double>(num_docs) / static_cast<double>(first));
+  const double rounds = std::max(1.0, std::ceil(std::log(all) / std::log(1.0 + static_cast<double>(growth))));
+  return {first, std::pow(all, 1.0 / rounds) - 1.0};
+}
+
+// Doc bounds of a schedule's rounds, aligned to bundles.  In the safe schedule
+// no round is larger than the candidate segments can always hold.
+std::vector<int64_t> round_bounds(const Schedule& sc, int64_t num_docs, bool safe) {
   // A safe round gives each workgroup at most one segment's worth of docs.
   static_assert(kSegmentSlots % kRoundAlign == 0, "safe rounds stay aligned");
-  const int64_t safe_step = kSegmentSlots;
-  const int64_t growth =
-      std::max<int64_t>(8, std::min(kSelectSlots / 2 / topk, kRoundCandidates / (num_queries * topk)));
-  const int64_t first = topk <= 64 ? 2048 : 8192;
-  while (pos < num_docs) {
-    int64_t step = safe ? safe_step : (pos == 0 ? first : growth * pos);
-    step = (step + kRoundAlign - 1) / kRoundAlign * kRoundAlign;
-    pos = std::min(num_docs, pos + step);
+  std::vector<int64_t> b{0};
+  for (int64_t pos = 0; pos < num_docs;) {
+    const int64_t step = safe ? kSegmentSlots
+                         : pos == 0
+                             ? sc.first
+                             : std::max<int64_t>(1, static_cast<int64_t>(std::ceil(sc.growth * static_cast<double>(pos))));
+    pos = std::min(num_docs, pos + (step + kRoundAlign - 1) / kRoundAlign * kRoundAlign);
     b.push_back(pos);
   }
   return b;
@@ -877,7 +895,7 @@ extern "C" int st_filtered_topk(const int64_t* packed, int64_t num_queries,
 
     for (int attempt = 0; attempt < 2; ++attempt) {
       const bool safe = attempt == 1;
-      const std::vector<int64_t> bounds = round_bounds(num_docs, num_queries, topk, safe);
+      const std::vector<int64_t> bounds = round_bounds(first_schedule(few, num_queries, num_docs, topk), num_docs, safe);
       for (size_t r = 0; r + 1 < bounds.size(); ++r) {
         state.first_round = r == 0 ? 1 : 0;
         const int nseg = score(emb, qv, m64, num_columns, num_queries, bounds[r], bounds[r + 1],
