@@ -95,7 +95,7 @@ def test_topk_random(dim, n, q, topk, density):
 
 
 def test_topk_rounds_and_query_chunks():
-    """60k docs cross several selection rounds (first round 8192 docs, then
+    """60k docs cross several selection rounds (first round 8,192 docs, then
     x8), each keeping the best 100 of its candidates; 600 queries cross the
     512 queries one launch of the dim-128 kernel scores."""
     rng = np.random.default_rng(7)
@@ -106,21 +106,54 @@ def test_topk_rounds_and_query_chunks():
     _check(ids[560:], sc[560:], emb32, qv32[560:], packed[560:], 60000, 100)
 
 
-@pytest.mark.parametrize("dim", [64, 128, 256])
-def test_topk_ties_overflow_and_safe_rounds(dim):
-    """All scores equal: the second round sends every doc past the threshold
-    (ties are kept), overflowing the candidate segments, so the selection is
-    redone with small rounds; the answer is the lowest ids."""
-    n, q = 50000, 3
+@pytest.mark.parametrize("dim,q", [(64, 3), (128, 3), (256, 3), (64, 150), (128, 150), (256, 150), (128, 600)])
+@pytest.mark.parametrize("n,topk", [(50000, 100), (50000, 1), (50000, 1000), (200_000, 100)])
+def test_topk_ties_overflow_and_safe_rounds(dim, q, n, topk):
+    """All scores equal: a later round sends every doc past the threshold (ties
+    are kept), overflowing the candidate segments, so the selection goes on from
+    there with small rounds; the answer is the lowest ids.  With 50,000 docs and
+    top 1 or 100 the round in the middle overflows and not the last; 150 queries
+    take the staged kernel, 600 two launches of it a round."""
     emb_bf = torch.ones((n, dim), dtype=torch.bfloat16)
     qv_bf = torch.ones((q, dim), dtype=torch.bfloat16)
     cols = (n + 2047) // 2048 * 32
     packed = np.full((q, cols), -1, dtype=np.int64)
     packed[1, :] = 0  # one query with an empty filter
-    H.note("[topk] all ties, overflow")
-    ids, sc = _gpu_topk(packed, emb_bf, qv_bf, n, 100)
-    assert ids[0].tolist() == list(range(100)) and ids[2].tolist() == list(range(100))
-    assert (sc[0] == dim).all() and (ids[1] == -1).all() and np.isneginf(sc[1]).all()
+    H.note(f"[topk] all ties, overflow dim={dim} q={q} n={n} topk={topk}")
+    ids, sc = _gpu_topk(packed, emb_bf, qv_bf, n, topk)
+    rest = np.arange(q) != 1
+    assert (ids[rest] == np.arange(topk)).all()
+    assert (sc[rest] == dim).all() and (ids[1] == -1).all() and np.isneginf(sc[1]).all()
+
+
+@pytest.mark.parametrize("q", [3, 150])
+@pytest.mark.parametrize("order", ["rising", "hole", "late", "blocks"])
+@pytest.mark.parametrize("topk", [1, 10, 100])
+def test_topk_ordered_docs_vs_oracle(q, order, topk):
+    """Docs in an order by which the first ones say nothing of the rest, each
+    overflowing one round or several: scores that rise all along, filters that
+    pass nothing at first (for all queries, or for one), docs of one kind in
+    blocks.  Queries that did not overflow are redone with the others."""
+    n, dim = 150_000, 64
+    rng = np.random.default_rng(q + topk)
+    emb_bf, qv_bf, emb32, qv32, packed = _random_case(rng, n, dim, q, 0.9)
+    if order == "rising":
+        level = (np.arange(n) // 700).astype(np.float32)  # whole numbers: exact in bf16 up to 256
+        emb_bf = _bf16(np.repeat(level[:, None], dim, 1))
+        qv_bf = _bf16(np.abs(rng.integers(1, 4, (q, dim))).astype(np.float32))
+    elif order == "hole":
+        packed[:, :1700] = 0
+    elif order == "late":
+        packed[q - 1, :300] = 0
+    else:
+        kind = rng.normal(0, 1, (50, dim))
+        emb_bf = _bf16(kind[np.arange(n) * 50 // n] * 0.3 + rng.normal(0, 0.03, (n, dim)))
+        qv_bf = _bf16(kind[rng.integers(0, 50, q)])
+    emb32, qv32 = emb_bf.float().numpy(), qv_bf.float().numpy()
+    H.note(f"[topk ordered] {order} q={q} topk={topk}")
+    ids, sc = _gpu_topk(packed, emb_bf, qv_bf, n, topk)
+    for at in (slice(0, 3), slice(q - 2, q)):
+        _check(ids[at], sc[at], emb32, qv32[at], packed[at], n, topk)
 
 
 @pytest.mark.parametrize("dim", [64, 128, 256])
