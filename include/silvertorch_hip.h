@@ -358,7 +358,7 @@ int st_bloom_compact_ids(const int64_t* packed, int64_t num_queries,
  * 16-byte aligned with at least num_docs rows.  workspace: device memory of
  * st_filtered_topk_workspace_bytes(num_queries) bytes.  Synchronises the
  * stream once (to learn whether a candidate list overflowed; if one did, the
- * selection is redone with smaller rounds).
+ * selection goes on from there with smaller rounds, and waits again).
  * ------------------------------------------------------------------------- */
 int64_t st_filtered_topk_workspace_bytes(int64_t num_queries);
 int st_filtered_topk(const int64_t* packed, int64_t num_queries,
